@@ -487,32 +487,76 @@ bool gemm_supported(int64_t m, int64_t n, int64_t k, int bits, int bs, bool has_
     if (m <= 0 || n <= 0 || (bits != 4 && bits != 8) || k <= 0 || k % kKS) return false;
     if (bs != 16 && bs != 32 && bs != 64 && bs != 128) return false;
     if (k % bs) return false;
-    const int64_t bpc = k / bs;
-    // The scale and zero-point dwords of the last column must not reach past the arrays.
-    if (bs > 32 && (n * bpc) % 2) return false;
-    const int64_t zpb = bits == 8 ? bpc : (bpc + 1) / 2;
-    if (has_zp && (n * zpb) % 4) return false;
-    // The DMA sources are a uniform base plus a 32-bit byte offset per lane.
+    // The sources are a base plus a 32-bit byte offset per lane.
     if (m * k * 2 >= (int64_t)1 << 32 || n * k * bits / 8 >= (int64_t)1 << 32) return false;
-    return true;
+    // Blocks of 16: the zero-point dword of the last column must not reach past the array.
+    const int64_t zpb = bits == 8 ? k / bs : (k / bs + 1) / 2;
+    return bs != 16 || !has_zp || (n * zpb) % 4 == 0;
 }
 
-GemmConfig gemm_config(int64_t m, int64_t n, int64_t k) {
-    GemmConfig c{};
-    c.bm = kBM;
-    c.bn = kBN;
-    c.tiles_m = (m + kBM - 1) / kBM;
-    c.tiles_n = (n + kBN - 1) / kBN;
-    // Fewer tiles than the 256 CUs (M = 256: 64 tiles of 8192 columns): split K over up to four
-    // workgroups per tile, each split at least eight 64-k steps and none empty.
-    const int64_t tiles = c.tiles_m * c.tiles_n;
-    const int64_t steps = k / kKS;
-    int ks = 1;
-    if (tiles < 256 && (m * n) % 4 == 0)
-        ks = (int)std::max<int64_t>(1, std::min<int64_t>({4, 256 / tiles, steps / 8}));
-    while (ks > 1 && ((steps + ks - 1) / ks) * (ks - 1) >= steps) --ks;
-    c.ksplit = ks;
-    return c;
+GemmConfig gemm_config(int64_t m, int64_t n, int64_t k, int bits, int bs) {
+    auto tiled = [&](int tile, int bm, int bn, int waves) {
+        return GemmConfig{tile, bm, bn, waves, (m + bm - 1) / bm, (n + bn - 1) / bn, 1};
+    };
+    const bool can_split = (m * n) % 4 == 0;
+    if (bs == 16) {
+        GemmConfig c = tiled(kTile256x128, 256, 128, 8);
+        // Fewer tiles than the 256 CUs: split K over up to four workgroups per tile, each split
+        // at least eight 64-k steps and none empty.
+        const int64_t tiles = c.tiles_m * c.tiles_n;
+        const int64_t steps = k / kKS;
+        int ks = 1;
+        if (tiles < 256 && can_split)
+            ks = (int)std::max<int64_t>(1, std::min<int64_t>({4, 256 / tiles, steps / 8}));
+        while (ks > 1 && ((steps + ks - 1) / ks) * (ks - 1) >= steps) --ks;
+        c.ksplit = ks;
+        return c;
+    }
+    // The tile and K split with the least estimated time: rounds of resident workgroups (one of
+    // the 8-wavefront tile per CU, two of the others) times the quads of a split times the time
+    // per quad, measured at M = 100-2048 on the Phi-3.5-mini nodes with the CU full and with one
+    // workgroup on it; a split adds the partials' traffic and the launch that sums them.  The
+    // widest tile is first: another one has to be a twentieth better.  E.g. qkv at M = 2048 (3072 x
+    // 9216: 576 tiles of 128 x 256, 2.25 rounds) takes 128 x 192, 768 workgroups in 1.5 rounds of
+    // two: 136 us against 184; 100 rows of 3072 x 3072 take 64 x 128 split four ways, 10.8 us
+    // against 20.0 on 128 x 256; 256 rows of 3072 x 8192 keep 128 x 256, 25.4 us against 29.3.
+    struct Cost {
+        int tile, bm, bn, waves;
+        double full, lone;                               // us per quad: CU full, one workgroup
+    };
+    const Cost costs[] = {{kTile128x256, 128, 256, 8, 2.5, 2.5},
+                          {kTile128x192, 128, bits == 8 ? 128 : 192, 4, bits == 8 ? 2.6 : 3.4,
+                           bits == 8 ? 1.9 : 2.3},
+                          {kTile64x128, 64, 128, 4, 1.7, 1.1}};
+    const int64_t quads = (k + 127) / 128;
+    GemmConfig best{};
+    double best_us = 0.0;
+    for (const Cost& t : costs) {
+        GemmConfig c = tiled(t.tile, t.bm, t.bn, t.waves);
+        GemmConfig own{};
+        double own_us = 0.0;
+        for (int ks = 1; ks <= (can_split ? 4 : 1); ++ks) {
+            const int64_t per = ((quads + ks - 1) / ks + 1) & ~(int64_t)1;   // pairs of quads
+            if (ks > 1 && (quads / ks < 4 || per * (ks - 1) >= quads)) continue;
+            const int64_t items = c.tiles_m * c.tiles_n * ks;
+            const int64_t resident = t.waves == 8 ? 256 : 512;
+            const int64_t rest = items % resident;
+            double us = (double)(items / resident) * t.full +
+                        (rest == 0 ? 0.0 : rest <= 256 ? t.lone : t.full);
+            us *= (double)std::min(per, quads);
+            if (ks > 1) us += 2.0 + 8.0 * ks * (double)m * (double)n / 7e6;
+            if (own_us == 0.0 || us < own_us) {
+                own = c;
+                own.ksplit = ks;
+                own_us = us;
+            }
+        }
+        if (best_us == 0.0 || own_us < 0.95 * best_us) {
+            best = own;
+            best_us = own_us;
+        }
+    }
+    return best;
 }
 
 size_t gemm_workspace_bytes(const GemmConfig& c, int64_t m, int64_t n) {
@@ -546,25 +590,12 @@ static hipError_t gemm_zp(const GemmConfig& c, const void* a, const uint8_t* b, 
     return gemm_go<BITS, BS, false>(c, a, b, s, z, y, m, n, k, part, st);
 }
 
-template <int BITS>
-static hipError_t gemm_bs(int bs, const GemmConfig& c, const void* a, const uint8_t* b,
-                          const void* s, const uint8_t* z, void* y, int64_t m, int64_t n,
-                          int64_t k, float* part, hipStream_t st) {
-    switch (bs) {
-        case 16: return gemm_zp<BITS, 16>(c, a, b, s, z, y, m, n, k, part, st);
-        case 32: return gemm_zp<BITS, 32>(c, a, b, s, z, y, m, n, k, part, st);
-        case 64: return gemm_zp<BITS, 64>(c, a, b, s, z, y, m, n, k, part, st);
-        case 128: return gemm_zp<BITS, 128>(c, a, b, s, z, y, m, n, k, part, st);
-        default: return hipErrorInvalidValue;
-    }
-}
-
-hipError_t launch_gemm_cfg(const GemmConfig& c, const void* a, const uint8_t* b, const void* s,
-                           const uint8_t* z, void* y, int64_t m, int64_t n, int64_t k, int bits,
-                           int bs, hipStream_t st, void* workspace, size_t workspace_bytes) {
+hipError_t launch_gemm(const void* a, const uint8_t* b, const void* s, const uint8_t* z, void* y,
+                       int64_t m, int64_t n, int64_t k, int bits, int bs, hipStream_t st,
+                       void* workspace, size_t workspace_bytes, const uint8_t* b_strips) {
     if (m == 0) return hipSuccess;
     if (!gemm_supported(m, n, k, bits, bs, z != nullptr)) return hipErrorInvalidValue;
-    if (c.bm != kBM || c.bn != kBN || c.ksplit < 1) return hipErrorInvalidValue;
+    const GemmConfig c = gemm_config(m, n, k, bits, bs);
     // the K split needs the partial buffer and 8-byte aligned output; without them, one pass
     const size_t need = gemm_workspace_bytes(c, m, n);
     float* part = need && workspace && workspace_bytes >= need &&
@@ -572,15 +603,12 @@ hipError_t launch_gemm_cfg(const GemmConfig& c, const void* a, const uint8_t* b,
                           reinterpret_cast<uintptr_t>(y) % 8 == 0
                       ? static_cast<float*>(workspace)
                       : nullptr;
-    return bits == 8 ? gemm_bs<8>(bs, c, a, b, s, z, y, m, n, k, part, st)
-                     : gemm_bs<4>(bs, c, a, b, s, z, y, m, n, k, part, st);
-}
-
-hipError_t launch_gemm(const void* a, const uint8_t* b, const void* s, const uint8_t* z, void* y,
-                       int64_t m, int64_t n, int64_t k, int bits, int bs, hipStream_t st,
-                       void* workspace, size_t workspace_bytes) {
-    return launch_gemm_cfg(gemm_config(m, n, k), a, b, s, z, y, m, n, k, bits, bs, st, workspace,
-                           workspace_bytes);
+    if (bs == 16)
+        return bits == 8 ? gemm_zp<8, 16>(c, a, b, s, z, y, m, n, k, part, st)
+                         : gemm_zp<4, 16>(c, a, b, s, z, y, m, n, k, part, st);
+    if (bits == 8) return launch_gemm_direct_b8(bs, c, a, b, s, z, y, m, n, k, part, st);
+    return b_strips ? launch_gemm_direct_b4n(bs, c, a, b_strips, s, z, y, m, n, k, part, st)
+                    : launch_gemm_direct_b4(bs, c, a, b, s, z, y, m, n, k, part, st);
 }
 
 }  // namespace mnb

@@ -81,25 +81,37 @@ hipError_t launch_gemv_stream_cfg(const StreamConfig& c, const void* a, const ui
                                   const void* s, const uint8_t* z, void* y, int64_t m, int64_t n,
                                   int64_t k, int bits, int bs, hipStream_t stream);
 
-// Tile shape of the prefill GEMM (mnb_gemm.hip).
+// Tile shapes of the prefill GEMM: blocks of 32 and more (mnb_gemm_direct.hpp) in rows x columns
+// of a workgroup -- kTile128x192 is 128 x 128 for 8-bit weights, whose operands take twice the
+// registers -- and blocks of 16 (mnb_gemm.hip).
+enum GemmTile : int { kTile128x256 = 0, kTile128x192 = 1, kTile64x128 = 2, kTile256x128 = 3 };
 struct GemmConfig {
+    int tile;            // GemmTile
     int bm, bn;          // workgroup tile
+    int waves;           // wavefronts per workgroup
     int64_t tiles_m, tiles_n;
     int ksplit;          // workgroups per tile along K (fp32 partials summed by a second launch)
 };
 
 bool gemm_supported(int64_t m, int64_t n, int64_t k, int bits, int bs, bool has_zp);
-GemmConfig gemm_config(int64_t m, int64_t n, int64_t k);
+GemmConfig gemm_config(int64_t m, int64_t n, int64_t k, int bits, int bs);
 // fp32 partials of a K split (0 when the config does not split)
 size_t gemm_workspace_bytes(const GemmConfig& c, int64_t m, int64_t n);
 // With less workspace than gemm_workspace_bytes (or none) the launch runs without the K split.
+// b_strips: the MFMA-native strip copy of int4 weights (launch_strip_pack), read in place of b.
 hipError_t launch_gemm(const void* a, const uint8_t* b, const void* s, const uint8_t* z, void* y,
                        int64_t m, int64_t n, int64_t k, int bits, int bs, hipStream_t stream,
-                       void* workspace = nullptr, size_t workspace_bytes = 0);
-hipError_t launch_gemm_cfg(const GemmConfig& c, const void* a, const uint8_t* b, const void* s,
-                           const uint8_t* z, void* y, int64_t m, int64_t n, int64_t k, int bits,
-                           int bs, hipStream_t stream, void* workspace = nullptr,
-                           size_t workspace_bytes = 0);
+                       void* workspace = nullptr, size_t workspace_bytes = 0,
+                       const uint8_t* b_strips = nullptr);
+hipError_t launch_gemm_direct_b4(int bs, const GemmConfig& c, const void* a, const uint8_t* b,
+                                 const void* s, const uint8_t* z, void* y, int64_t m, int64_t n,
+                                 int64_t k, float* part, hipStream_t stream);
+hipError_t launch_gemm_direct_b4n(int bs, const GemmConfig& c, const void* a, const uint8_t* b,
+                                  const void* s, const uint8_t* z, void* y, int64_t m, int64_t n,
+                                  int64_t k, float* part, hipStream_t stream);
+hipError_t launch_gemm_direct_b8(int bs, const GemmConfig& c, const void* a, const uint8_t* b,
+                                 const void* s, const uint8_t* z, void* y, int64_t m, int64_t n,
+                                 int64_t k, float* part, hipStream_t stream);
 // Y = the sum of `ksplit` fp32 partial planes of m*n elements, in split order.
 hipError_t launch_splitk_sum(const float* part, void* y, int64_t mn, int ksplit,
                              hipStream_t stream);

@@ -246,8 +246,8 @@ static int plan_search(const mnb_problem* p, mnb_plan_info* out) {
         return MNB_OK;
     }
     if (kern == MNB_KERNEL_GEMM_MFMA) {
-        const mnb::GemmConfig c = mnb::gemm_config(p->m, p->n, p->k);
-        out->waves_per_group = 8;
+        const mnb::GemmConfig c = mnb::gemm_config(p->m, p->n, p->k, p->bits, p->block_size);
+        out->waves_per_group = c.waves;
         out->tile_n = c.bn;
         out->tile_m = c.bm;
         out->grid_x = c.tiles_m * c.tiles_n * c.ksplit;
@@ -383,13 +383,14 @@ static int matmul_impl(const mnb_problem* p, const void* a, const uint8_t* b,
                    ? MNB_KERNEL_STRIP_MFMA
                    : MNB_KERNEL_GROUP_MFMA;
     }
-    // The GEMM's LDS DMA also fetches scales and zero points as aligned dwords; the row-tiled
+    // The block-16 GEMM's LDS DMA also fetches scales and zero points as aligned dwords; the row-tiled
     // GEMV (int4, block >= 32), else the 16-row MFMA GEMV or the generic kernel, takes any other
     // case of the same form.
     if (kern == MNB_KERNEL_STRIP_MFMA && !mnb::strip_gemv_aligned(a, b, scales, zero_points, false))
         kern = MNB_KERNEL_GROUP_MFMA;
     if (kern == MNB_KERNEL_GEMM_MFMA && p->dtype == MNB_DTYPE_F16 &&
-        (!aligned(scales, 4) || !aligned(zero_points, 4) ||
+        ((p->block_size == 16 && (!aligned(scales, 4) || !aligned(zero_points, 4))) ||
+         !aligned(scales, 2) ||
          !mnb::gemm_supported(p->m, p->n, p->k, p->bits, p->block_size, zero_points != nullptr))) {
         if (mnb::group_gemv_supported(p->k, p->bits, p->block_size))
             kern = MNB_KERNEL_GROUP_MFMA;
@@ -424,7 +425,7 @@ static int matmul_impl(const mnb_problem* p, const void* a, const uint8_t* b,
     } else if (kern == MNB_KERNEL_GEMM_MFMA) {
         e = p->dtype == MNB_DTYPE_F16
                 ? mnb::launch_gemm(a, b, scales, zero_points, y, p->m, p->n, p->k, p->bits,
-                                   p->block_size, st, workspace, workspace_bytes)
+                                   p->block_size, st, workspace, workspace_bytes, b_strips)
                 : mnb::launch_gemm_f32(a, b, scales, zero_points, y, p->m, p->n, p->k, p->bits,
                                        p->block_size, st);
     } else if (kern == MNB_KERNEL_GEMV_STREAM) {

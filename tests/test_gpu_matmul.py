@@ -320,6 +320,74 @@ def test_gemm_parity(cuda, M, N, K, bits, bs, zp):
     _check_f16(y, ref, f"gemm M={M} N={N} K={K} bits={bits} bs={bs}")
 
 
+# One case or more per tile shape, weight width and block size of the direct-to-register GEMM: no
+# whole number of tiles in M or N, K with and without a last half quad (K % 128 == 64), an odd
+# number of quads, columns whose scales start at odd 2-byte offsets (K / bs odd) and zero points
+# at odd bytes; (rows, columns) of the tile the planner must take.
+DIRECT_SHAPES = [
+    (65, 130, 320, 4, 32, True, (64, 128)),
+    (127, 129, 448, 4, 64, True, (64, 128)),
+    (70, 250, 640, 4, 128, True, (64, 128)),
+    (91, 77, 704, 8, 64, True, (64, 128)),
+    (2001, 3050, 320, 4, 64, True, (128, 192)),
+    (2001, 3050, 384, 4, 32, True, (128, 192)),
+    (1999, 3041, 256, 4, 128, False, (128, 192)),
+    (2040, 8100, 192, 4, 32, True, (128, 256)),
+    (2040, 8101, 192, 4, 64, False, (128, 256)),
+    (2040, 8100, 128, 4, 128, True, (128, 256)),
+    (2040, 8101, 192, 8, 32, True, (128, 256)),
+    (2040, 6100, 320, 8, 64, True, (128, 128)),
+    (2040, 6100, 256, 8, 128, True, (128, 128)),
+]
+
+
+@pytest.mark.parametrize("layout", ["ort", "strips", "scales_off"])
+@pytest.mark.parametrize("M,N,K,bits,bs,zp,tile", DIRECT_SHAPES)
+def test_gemm_direct_tiles(cuda, M, N, K, bits, bs, zp, tile, layout):
+    """Every output against the fp64 product of the dequantised weights (the GPU's fp64 matmul), at
+    the bar of this file.  Layouts: ORT's; the strip copy of a prepacked node (where the node has
+    one); ORT's with scales that start 2 bytes off a dword."""
+    import ctypes as C
+    import mnb
+    import torch
+
+    p = mnb.problem(M, N, K, bits, bs, zp)
+    info = mnb.plan(p)
+    assert (info.kernel, info.tile_m, info.tile_n) == (mnb.KERNEL_GEMM_MFMA, *tile)
+    inp = orc.make_inputs(M, N, K, bits=bits, block_size=bs, with_zp=zp, seed=M + N + K)
+    t = {k: _dev(v, cuda) for k, v in inp.items() if v is not None}
+    print(f"[gpu] direct gemm {M}x{N}x{K} bits={bits} bs={bs} {layout}", flush=True)
+    if layout == "strips":
+        lib, s, w = mnb.load(), C.c_void_p(), C.c_void_p()
+        mnb.check(lib.mnb_session_create(0, C.byref(s)))
+        z = inp["zp"]
+        mnb.check(lib.mnb_weights_upload(
+            s, C.byref(p), inp["B"].ctypes.data, inp["B"].nbytes, inp["scales"].ctypes.data,
+            inp["scales"].nbytes, z.ctypes.data if zp else None, z.nbytes if zp else 0, C.byref(w)))
+        rc = lib.mnb_weights_prepack(w, None)
+        y = torch.empty(M, N, dtype=torch.float16, device=cuda)
+        torch.cuda.synchronize()
+        if rc == mnb.MNB_OK:
+            mnb.check(lib.mnb_session_run(s, w, M, t["A"].data_ptr(), 1, y.data_ptr(), 1))
+        mnb.check(lib.mnb_weights_release(w))
+        mnb.check(lib.mnb_session_destroy(s))
+        if rc == mnb.MNB_ERR_UNSUPPORTED:
+            pytest.skip("the node has no strip copy")
+        mnb.check(rc)
+    else:
+        sc = t["scales"].reshape(-1)
+        if layout == "scales_off":
+            sc = torch.cat([sc[:1], sc])[1:]
+            assert sc.data_ptr() % 4 == 2
+        y = mnb.matmul_nbits(t["A"], t["B"], sc, t.get("zp"), N, K, bits, bs)
+    torch.cuda.synchronize()
+    w64 = torch.from_numpy(orc.dequantize_f32(inp["B"], inp["scales"], inp["zp"], N, K, bits,
+                                             bs)
+                           .astype(np.float64)).to(cuda)
+    ref = (t["A"].double() @ w64.t()).cpu().numpy()
+    _check_f16(y.cpu().numpy(), ref, f"direct {M}x{N}x{K}")
+
+
 def test_gemm_uneven_k_split(cuda):
     """K split whose last split is shorter: K = 1600 is 25 steps of 64, over 3 workgroups per tile
     (9, 9 and 7 steps).  Checked against the oracle, and against the same GEMM run unsplit (no
