@@ -54,6 +54,7 @@ HIP_SOURCES = [
     CSRC / "kernels" / "mnb_gemm_direct_b4.hip",
     CSRC / "kernels" / "mnb_gemm_direct_b4n.hip",
     CSRC / "kernels" / "mnb_gemm_direct_b8.hip",
+    CSRC / "kernels" / "mnb_gemm_grouped.hip",
     CSRC / "kernels" / "mnb_gemm.hip",
     CSRC / "kernels" / "mnb_group_gemv.hip",
     CSRC / "kernels" / "mnb_strip_gemv.hip",

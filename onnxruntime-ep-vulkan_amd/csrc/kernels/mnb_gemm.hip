@@ -524,9 +524,10 @@ GemmConfig gemm_config(int64_t m, int64_t n, int64_t k, int bits, int bs) {
         int tile, bm, bn, waves;
         double full, lone;                               // us per quad: CU full, one workgroup
     };
+    const bool wide = bits == 4 && bs == 32;
     const Cost costs[] = {{kTile128x256, 128, 256, 8, 2.5, 2.5},
-                          {kTile128x192, 128, bits == 8 ? 128 : 192, 4, bits == 8 ? 2.6 : 3.4,
-                           bits == 8 ? 1.9 : 2.3},
+                          {kTile128x192, 128, wide ? 192 : 128, 4, wide ? 3.4 : 2.6,
+                           wide ? 2.3 : 1.9},
                           {kTile64x128, 64, 128, 4, 1.7, 1.1}};
     const int64_t quads = (k + 127) / 128;
     GemmConfig best{};

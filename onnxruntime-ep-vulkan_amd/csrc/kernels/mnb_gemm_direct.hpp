@@ -48,6 +48,61 @@ namespace {
 
 typedef __attribute__((address_space(3))) void* lds_void_ptr;
 
+// What a launch does: one dense problem; the expert-grouped problems of a mixture of experts; the
+// same with SwiGLU applied to interleaved (gate, linear) columns as they are stored.
+enum : int { kDense = 0, kGrouped = 1, kGroupedSwiglu = 2 };
+
+// The expert-grouped launch: expert e's rows are offsets[e] .. offsets[e + 1] - 1 of Y, each
+// multiplying row row_index[r] of A (row r itself without an index).
+struct DirectGroups {
+    const int32_t* offsets;      // [experts + 1]
+    const int32_t* row_index;    // or null
+    const f16* bias;             // SwiGLU: [experts][N] or null
+    int experts;
+    float alpha, beta, limit;
+    int has_limit;
+};
+
+template <int BM>
+__device__ __forceinline__ int group_tiles_of(const DirectGroups& g, int e) {
+    return e < g.experts ? (g.offsets[e + 1] - g.offsets[e] + BM - 1) / BM : 0;
+}
+
+// Row tiles of all experts: ceil(rows / BM) each.
+template <int BM>
+__device__ __forceinline__ int group_row_tiles(const DirectGroups& g, int lane) {
+    int n = 0;
+    for (int e = lane; e < g.experts; e += 64) n += group_tiles_of<BM>(g, e);
+    for (int d = 32; d > 0; d >>= 1) n += __shfl_xor(n, d);
+    return __builtin_amdgcn_readfirstlane(n);
+}
+
+// The expert that row tile `tile` belongs to (tile < group_row_tiles), the tile's first row and
+// the end of the expert's rows: 64 experts at a time, their tile counts summed along the lanes.
+template <int BM>
+__device__ __forceinline__ void group_tile(const DirectGroups& g, int tile, int lane, int* expert,
+                                           int* row0, int* row_end) {
+    int e0 = 0, seen = 0;
+    for (;; e0 += 64) {
+        int sum = group_tiles_of<BM>(g, e0 + lane);
+        const int own = sum;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int v = __shfl_up(sum, d);
+            if (lane >= d) sum += v;
+        }
+        const uint64_t past = __ballot(seen + sum > tile);
+        if (past || e0 + 64 >= g.experts) {
+            const int l = past ? __builtin_ctzll(past) : 63;
+            *expert = __builtin_amdgcn_readfirstlane(min(e0 + l, g.experts - 1));
+            const int before = __builtin_amdgcn_readfirstlane(__shfl(seen + sum - own, l));
+            *row0 = __builtin_amdgcn_readfirstlane(g.offsets[*expert]) + (tile - before) * BM;
+            *row_end = __builtin_amdgcn_readfirstlane(g.offsets[*expert + 1]);
+            return;
+        }
+        seen += __shfl(sum, 63);
+    }
+}
+
 // Buffer descriptor over `bytes` bytes (loads past them return zero).
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const void* p, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0,
@@ -75,13 +130,15 @@ __device__ __forceinline__ T load_any(const void* p) {
 
 // MT: 16-row tiles per workgroup; S: 16-column strips per wavefront; NW: wavefronts per workgroup,
 // side by side along N; NATIVE: B is the strip copy.
-template <int BITS, int BS, bool HAS_ZP, int MT, int S, int NW, bool NATIVE>
+template <int BITS, int BS, bool HAS_ZP, int MT, int S, int NW, bool NATIVE,
+          int MODE>
 __global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(2, 2)))
 gemm_direct(const f16* __restrict__ A, const uint8_t* __restrict__ B, const f16* __restrict__ Sc,
             const uint8_t* __restrict__ Z, f16* __restrict__ Y, int M, int N, int K, int tiles_m,
             int tiles_n, int ksplit, float* __restrict__ part,
-            uint32_t a_bytes) {
+            uint32_t a_bytes, DirectGroups grp) {
     static_assert(BITS == 4 || (BITS == 8 && !NATIVE), "form");
+    static_assert(MODE == kDense || (BITS == 4 && !HAS_ZP), "expert weights are symmetric int4");
     constexpr int CPB = BS / 32;                         // 32-k chunks per block
     constexpr int BPQ = 4 / CPB;                         // blocks per quad
     constexpr int kBM = 16 * MT;
@@ -97,6 +154,9 @@ gemm_direct(const f16* __restrict__ A, const uint8_t* __restrict__ B, const f16*
     const int nl = lane & 15;
     const int g = lane >> 4;
 
+    // Grouped: the row tiles are those of the experts in order, as many as their row counts (known
+    // on the device only) need; every wavefront counts them from the offsets.
+    if constexpr (MODE != kDense) tiles_m = group_row_tiles<kBM>(grp, lane);
     const int V = tiles_m * tiles_n * ksplit;
     const int per_xcd = (V + 7) >> 3;
     if ((int)(blockIdx.x >> 3) >= per_xcd) return;
@@ -106,12 +166,19 @@ gemm_direct(const f16* __restrict__ A, const uint8_t* __restrict__ B, const f16*
     const int split = item - tile * ksplit;
     const int tile_m = tile / tiles_n;
     const int tile_n = tile - tile_m * tiles_n;
-    const int m0 = tile_m * kBM;
+    int m0 = tile_m * kBM;
     const int bpc = K / BS;
     const int zpb = BITS == 8 ? bpc : (bpc + 1) >> 1;
     const int cb = K * BITS / 8;                         // bytes per column of B
     const int strips = (N + 15) >> 4;
     const int KQ = (K + 127) >> 7;
+    int expert = 0;
+    if constexpr (MODE != kDense) {
+        // M: the end of the expert's rows; B, Sc: its weights
+        group_tile<kBM>(grp, tile_m, lane, &expert, &m0, &M);
+        B += NATIVE ? (int64_t)expert * strips * KQ * 1024 : (int64_t)expert * N * cb;
+        Sc += (int64_t)expert * N * bpc;
+    }
     const int strip0 = (tile_n * NW + wave) * S;
     const bool active = strip0 < strips;                 // else: only its share of the A loads
     const int per_split = ((KQ + ksplit - 1) / ksplit + 1) & ~1;   // pairs of quads
@@ -126,10 +193,14 @@ gemm_direct(const f16* __restrict__ A, const uint8_t* __restrict__ B, const f16*
         const int row = 4 * (AI * wave + j) + (lane >> 4);
         int gm = m0 + row;
         gm = gm < M ? gm : M - 1;                        // clamped rows are never stored
+        if constexpr (MODE != kDense) {
+            if (grp.row_index) gm = grp.row_index[gm];
+        }
         a_off[j] = (uint32_t)(((int64_t)gm * K + 8 * (a_slot ^ (row & 15))) * 2);
     }
     const auto ra = buffer_of(A, a_bytes);
-    auto issue_a = [&](int q) {
+    auto issue_a = [&](int q, int rows) {                // the wavefronts whose rows are needed
+        if (4 * AI * wave >= rows) return;
         uint8_t* dst = smem + (q & 1) * kStage + wave * AI * 1024;
 #pragma unroll
         for (int j = 0; j < AI; ++j)
@@ -224,179 +295,224 @@ gemm_direct(const f16* __restrict__ A, const uint8_t* __restrict__ B, const f16*
         }
     };
 
-    f32x4 acc[MT][S];
+    // The K loop and the stores over the first MV row tiles.
+    auto body = [&](auto mt_c) {
+        constexpr int MV = decltype(mt_c)::value;
+        f32x4 acc[MV][S];
 #pragma unroll
-    for (int i = 0; i < MT; ++i)
+        for (int i = 0; i < MV; ++i)
 #pragma unroll
-        for (int t = 0; t < S; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < S; ++t) acc[i][t] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    // the lane part of the A operand reads: row 16 i + nl, chunk c, 16-byte slot 4 c + g
-    int a_lane[4];
+        // the lane part of the A operand reads: row 16 i + nl, chunk c, 16-byte slot 4 c + g
+        int a_lane[4];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) a_lane[c] = nl * 256 + (((4 * c + g) ^ nl) << 4);
+        for (int c = 0; c < 4; ++c) a_lane[c] = nl * 256 + (((4 * c + g) ^ nl) << 4);
 
-    // half: which quad of the pair
-    auto compute = [&](const u32x4 (&rw)[S][WPL], const Pair& r, int q, auto half_c) {
-        constexpr int half = decltype(half_c)::value;
-        const uint8_t* base = smem + (q & 1) * kStage;
-        // the operand dwords of each chunk: dword g of the chunk (8-bit: dwords 2g and 2g + 1)
-        uint32_t wv[S][WPL][4];
-#pragma unroll
-        for (int t = 0; t < S; ++t) {
-            if constexpr (BITS == 4) {
-                wv[t][0][0] = rw[t][0].x;
-                wv[t][0][1] = rw[t][0].y;
-                wv[t][0][2] = rw[t][0].z;
-                wv[t][0][3] = rw[t][0].w;
-            } else {
-                wv[t][0][0] = rw[t][0].x;
-                wv[t][WPL - 1][0] = rw[t][0].y;
-                wv[t][0][1] = rw[t][0].z;
-                wv[t][WPL - 1][1] = rw[t][0].w;
-                wv[t][0][2] = rw[t][WPL - 1].x;
-                wv[t][WPL - 1][2] = rw[t][WPL - 1].y;
-                wv[t][0][3] = rw[t][WPL - 1].z;
-                wv[t][WPL - 1][3] = rw[t][WPL - 1].w;
-            }
-            if constexpr (!NATIVE) {
-#pragma unroll
-                for (int h = 0; h < WPL; ++h)
-                    transpose_rows(wv[t][h][0], wv[t][h][1], wv[t][h][2], wv[t][h][3]);
-            }
-        }
-        const int blocks = min(BPQ, ((K >> 5) - 4 * q) / CPB);
-        constexpr int AH = 3;                            // operand reads in flight
-        f16x8 a[AH][CPB];
-        auto read_a = [&](int f) {                       // f = block * MT + row tile
-#pragma unroll
-            for (int cc = 0; cc < CPB; ++cc)
-                a[f % AH][cc] = *reinterpret_cast<const f16x8*>(
-                    base + a_lane[(f / MT) * CPB + cc] + 4096 * (f % MT));
-        };
-#pragma unroll
-        for (int f = 0; f < AH; ++f) read_a(f);
-        f32x4 p[2][S];
-        float psc[S];
-#pragma unroll
-        for (int t = 0; t < S; ++t) psc[t] = 0.f;
-        auto retire = [&](int f, int t) {                // tile f's partial of strip t, scaled
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-                acc[f % MT][t][e] = __builtin_fmaf(p[f & 1][t][e], psc[t], acc[f % MT][t][e]);
-        };
-#pragma unroll
-        for (int bq = 0; bq < BPQ; ++bq) {
-            if (bq >= blocks) break;                     // uniform: the missing half of a quad
-            f16x8 bop[S][CPB];
-            float sc[S];
+        // half: which quad of the pair
+        auto compute = [&](const u32x4 (&rw)[S][WPL], const Pair& r, int q, auto half_c) {
+            constexpr int half = decltype(half_c)::value;
+            const uint8_t* base = smem + (q & 1) * kStage;
+            // the operand dwords of each chunk: dword g of the chunk (8-bit: dwords 2g and 2g + 1)
+            uint32_t wv[S][WPL][4];
 #pragma unroll
             for (int t = 0; t < S; ++t) {
-                const int bi = half * BPQ + bq;          // block of the pair
-                const uint32_t sw = r.sc[t][bi >> 1];
-                sc[t] = (float)__builtin_bit_cast(f16, (uint16_t)(bi & 1 ? sw >> 16 : sw & 0xFFFFu));
-                asm volatile("" : "+v"(sc[t]));
-                uint32_t z = 1u << (BITS - 1);
-                if constexpr (HAS_ZP)
-                    z = __builtin_amdgcn_ubfe(r.z[t][BITS == 8 ? bi >> 2 : 0],
-                                              BITS == 8 ? 8 * (bi & 3) : 4 * bi, BITS);
+                if constexpr (BITS == 4) {
+                    wv[t][0][0] = rw[t][0].x;
+                    wv[t][0][1] = rw[t][0].y;
+                    wv[t][0][2] = rw[t][0].z;
+                    wv[t][0][3] = rw[t][0].w;
+                } else {
+                    wv[t][0][0] = rw[t][0].x;
+                    wv[t][WPL - 1][0] = rw[t][0].y;
+                    wv[t][0][1] = rw[t][0].z;
+                    wv[t][WPL - 1][1] = rw[t][0].w;
+                    wv[t][0][2] = rw[t][WPL - 1].x;
+                    wv[t][WPL - 1][2] = rw[t][WPL - 1].y;
+                    wv[t][0][3] = rw[t][WPL - 1].z;
+                    wv[t][WPL - 1][3] = rw[t][WPL - 1].w;
+                }
+                if constexpr (!NATIVE) {
 #pragma unroll
-                for (int cc = 0; cc < CPB; ++cc) {
-                    const uint32_t w = wv[t][0][bq * CPB + cc];
-                    if constexpr (BITS == 8) {
-                        const uint32_t w1 = wv[t][WPL - 1][bq * CPB + cc];
-                        const f16x2 zo = as_h2(0xE400E400u + z * 0x10001u);   // -(1024 + z) twice
-                        bop[t][cc].s01 = byte_pair_lo(w, zo);
-                        bop[t][cc].s23 = byte_pair_hi(w, zo);
-                        bop[t][cc].s45 = byte_pair_lo(w1, zo);
-                        bop[t][cc].s67 = byte_pair_hi(w1, zo);
-                    } else if constexpr (NATIVE) {
-                        bop[t][cc] = native_pairs(w, as_h2(0xE400E400u + z * 0x10001u),
-                                                  as_h2(0xD400D400u + z * 0x100010u));
-                    } else {
-                        const f16x2 zo = zoff4((int)z);
-                        bop[t][cc].s01 = nib_pair<0>(w, zo);
-                        bop[t][cc].s23 = nib_pair<1>(w, zo);
-                        bop[t][cc].s45 = nib_pair<2>(w, zo);
-                        bop[t][cc].s67 = nib_pair<3>(w, zo);
+                    for (int h = 0; h < WPL; ++h)
+                        transpose_rows(wv[t][h][0], wv[t][h][1], wv[t][h][2], wv[t][h][3]);
+                }
+            }
+            const int blocks = min(BPQ, ((K >> 5) - 4 * q) / CPB);
+            constexpr int AH = 3 < MV ? 3 : MV;                            // operand reads in flight
+            f16x8 a[AH][CPB];
+            auto read_a = [&](int f) {                       // f = block * MV + row tile
+#pragma unroll
+                for (int cc = 0; cc < CPB; ++cc)
+                    a[f % AH][cc] = *reinterpret_cast<const f16x8*>(
+                        base + a_lane[(f / MV) * CPB + cc] + 4096 * (f % MV));
+            };
+#pragma unroll
+            for (int f = 0; f < AH; ++f) read_a(f);
+            f32x4 p[2][S];
+            float psc[S];
+#pragma unroll
+            for (int t = 0; t < S; ++t) psc[t] = 0.f;
+            auto retire = [&](int f, int t) {                // tile f's partial of strip t, scaled
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    acc[f % MV][t][e] = __builtin_fmaf(p[f & 1][t][e], psc[t], acc[f % MV][t][e]);
+            };
+#pragma unroll
+            for (int bq = 0; bq < BPQ; ++bq) {
+                if (bq >= blocks) break;                     // uniform: the missing half of a quad
+                f16x8 bop[S][CPB];
+                float sc[S];
+#pragma unroll
+                for (int t = 0; t < S; ++t) {
+                    const int bi = half * BPQ + bq;          // block of the pair
+                    const uint32_t sw = r.sc[t][bi >> 1];
+                    sc[t] = (float)__builtin_bit_cast(f16, (uint16_t)(bi & 1 ? sw >> 16 : sw & 0xFFFFu));
+                    asm volatile("" : "+v"(sc[t]));
+                    uint32_t z = 1u << (BITS - 1);
+                    if constexpr (HAS_ZP)
+                        z = __builtin_amdgcn_ubfe(r.z[t][BITS == 8 ? bi >> 2 : 0],
+                                                  BITS == 8 ? 8 * (bi & 3) : 4 * bi, BITS);
+#pragma unroll
+                    for (int cc = 0; cc < CPB; ++cc) {
+                        const uint32_t w = wv[t][0][bq * CPB + cc];
+                        if constexpr (BITS == 8) {
+                            const uint32_t w1 = wv[t][WPL - 1][bq * CPB + cc];
+                            const f16x2 zo = as_h2(0xE400E400u + z * 0x10001u);   // -(1024 + z) twice
+                            bop[t][cc].s01 = byte_pair_lo(w, zo);
+                            bop[t][cc].s23 = byte_pair_hi(w, zo);
+                            bop[t][cc].s45 = byte_pair_lo(w1, zo);
+                            bop[t][cc].s67 = byte_pair_hi(w1, zo);
+                        } else if constexpr (NATIVE) {
+                            bop[t][cc] = native_pairs(w, as_h2(0xE400E400u + z * 0x10001u),
+                                                      as_h2(0xD400D400u + z * 0x100010u));
+                        } else {
+                            const f16x2 zo = zoff4((int)z);
+                            bop[t][cc].s01 = nib_pair<0>(w, zo);
+                            bop[t][cc].s23 = nib_pair<1>(w, zo);
+                            bop[t][cc].s45 = nib_pair<2>(w, zo);
+                            bop[t][cc].s67 = nib_pair<3>(w, zo);
+                        }
+                    }
+                }
+#pragma unroll
+                for (int i = 0; i < MV; ++i) {
+                    const int f = bq * MV + i;
+#pragma unroll
+                    for (int t = 0; t < S; ++t) {
+                        f32x4 c = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                        for (int cc = 0; cc < CPB; ++cc)
+                            c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[f % AH][cc], bop[t][cc], c, 0, 0, 0);
+                        p[f & 1][t] = c;
+                        if (f > 0) retire(f - 1, t);
+                        if (i == 0) psc[t] = sc[t];
+                        if (t == S - 1 && f + AH < BPQ * MV) read_a(f + AH);
                     }
                 }
             }
 #pragma unroll
-            for (int i = 0; i < MT; ++i) {
-                const int f = bq * MT + i;
+            for (int t = 0; t < S; ++t) retire(BPQ * MV - 1, t);
+        };
+
+        // Quads in pairs from an even one: (A, w) one quad ahead, a pair's scales one pair ahead.
+        u32x4 w0[S][WPL], w1[S][WPL];
+        Pair p0, p1;
+        auto step = [&](int q, u32x4 (&now)[S][WPL], u32x4 (&next)[S][WPL], const Pair& p,
+                        Pair& pn, auto half) {
+            __builtin_amdgcn_s_waitcnt(0x7 << 4);            // vmcnt(0) lgkmcnt(0)
+            wg_barrier();
+            if (q + 1 < q1) {
+                issue_a(q + 1, 16 * MV);
+                load_w(next, q + 1);
+                if constexpr (decltype(half)::value == 0) {
+                    if (q + 2 < q1) load_p(pn, q + 2);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (active) compute(now, p, q, half);
+        };
+        using H0 = std::integral_constant<int, 0>;
+        using H1 = std::integral_constant<int, 1>;
+        issue_a(q0, 16 * MV);
+        load_w(w0, q0);
+        load_p(p0, q0);
+        for (int q = q0; q < q1; q += 4) {
+            step(q, w0, w1, p0, p1, H0{});
+            if (q + 1 >= q1) break;
+            step(q + 1, w1, w0, p0, p1, H1{});
+            if (q + 2 >= q1) break;
+            step(q + 2, w0, w1, p1, p0, H0{});
+            if (q + 3 >= q1) break;
+            step(q + 3, w1, w0, p1, p0, H1{});
+        }
+        if (!active) return;
+
+        if constexpr (MODE == kGroupedSwiglu) {
+            // Columns 2i, 2i + 1 are neighbouring lanes.  Of each pair of rows the even lane takes
+            // the first and the odd lane the second: it hands over its own half of the other row.
+            const bool odd = lane & 1;
 #pragma unroll
-                for (int t = 0; t < S; ++t) {
-                    f32x4 c = {0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < S; ++t) {
+                const int col = 16 * (strip0 + t) + (nl & ~1);
+                float bg = 0.f, bl = 0.f;
+                if (grp.bias && col < N) {
+                    const f16x2 b = *reinterpret_cast<const f16x2*>(grp.bias + (int64_t)expert * N + col);
+                    bg = (float)b.x;
+                    bl = (float)b.y;
+                }
 #pragma unroll
-                    for (int cc = 0; cc < CPB; ++cc)
-                        c = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[f % AH][cc], bop[t][cc], c, 0, 0, 0);
-                    p[f & 1][t] = c;
-                    if (f > 0) retire(f - 1, t);
-                    if (i == 0) psc[t] = sc[t];
-                    if (t == S - 1 && f + AH < BPQ * MT) read_a(f + AH);
+                for (int i = 0; i < MV; ++i)
+#pragma unroll
+                    for (int e = 0; e < 4; e += 2) {
+                        const float own = odd ? acc[i][t][e + 1] : acc[i][t][e];
+                        const float got = dpp_f<0xB1>(odd ? acc[i][t][e] : acc[i][t][e + 1]);
+                        // h is rounded to fp16 before its bias, as where h is stored
+                        float gt = (float)(f16)(odd ? got : own) + bg;
+                        float lt = (float)(f16)(odd ? own : got) + bl;
+                        if (grp.has_limit) {
+                            gt = fminf(gt, grp.limit);
+                            lt = fminf(fmaxf(lt, -grp.limit), grp.limit);
+                        }
+                        const float a = gt / (1.f + expf(-grp.alpha * gt)) * (lt + grp.beta);
+                        const int row = m0 + 16 * i + 4 * g + e + (odd ? 1 : 0);
+                        if (row < M && col < N) Y[(int64_t)row * (N >> 1) + (col >> 1)] = (f16)a;
+                    }
+            }
+            return;
+        }
+        float* const pbase = part ? part + (int64_t)split * M * N : nullptr;
+#pragma unroll
+        for (int i = 0; i < MV; ++i) {
+#pragma unroll
+            for (int t = 0; t < S; ++t) {
+                const int col = 16 * (strip0 + t) + nl;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int row = m0 + 16 * i + 4 * g + e;
+                    if (row < M && col < N) {
+                        if (MODE == kDense && pbase) pbase[(int64_t)row * N + col] = acc[i][t][e];
+                        else Y[(int64_t)row * N + col] = (f16)acc[i][t][e];
+                    }
                 }
             }
         }
-#pragma unroll
-        for (int t = 0; t < S; ++t) retire(BPQ * MT - 1, t);
     };
-
-    // Quads in pairs from an even one: (A, w) one quad ahead, a pair's scales one pair ahead.
-    u32x4 w0[S][WPL], w1[S][WPL];
-    Pair p0, p1;
-    auto step = [&](int q, u32x4 (&now)[S][WPL], u32x4 (&next)[S][WPL], const Pair& p,
-                    Pair& pn, auto half) {
-        __builtin_amdgcn_s_waitcnt(0x7 << 4);            // vmcnt(0) lgkmcnt(0)
-        wg_barrier();
-        if (q + 1 < q1) {
-            issue_a(q + 1);
-            load_w(next, q + 1);
-            if constexpr (decltype(half)::value == 0) {
-                if (q + 2 < q1) load_p(pn, q + 2);
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        if (active) compute(now, p, q, half);
-    };
-    using H0 = std::integral_constant<int, 0>;
-    using H1 = std::integral_constant<int, 1>;
-    issue_a(q0);
-    load_w(w0, q0);
-    load_p(p0, q0);
-    for (int q = q0; q < q1; q += 4) {
-        step(q, w0, w1, p0, p1, H0{});
-        if (q + 1 >= q1) break;
-        step(q + 1, w1, w0, p0, p1, H1{});
-        if (q + 2 >= q1) break;
-        step(q + 2, w0, w1, p1, p0, H0{});
-        if (q + 3 >= q1) break;
-        step(q + 3, w1, w0, p1, p0, H1{});
-    }
-    if (!active) return;
-
-    float* const pbase = part ? part + (int64_t)split * M * N : nullptr;
-#pragma unroll
-    for (int i = 0; i < MT; ++i) {
-#pragma unroll
-        for (int t = 0; t < S; ++t) {
-            const int col = 16 * (strip0 + t) + nl;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int row = m0 + 16 * i + 4 * g + e;
-                if (row < M && col < N) {
-                    if (pbase) pbase[(int64_t)row * N + col] = acc[i][t][e];
-                    else Y[(int64_t)row * N + col] = (f16)acc[i][t][e];
-                }
-            }
-        }
+    if constexpr (MODE == kDense) {
+        body(std::integral_constant<int, MT>{});
+    } else {
+        // experts leave tiles part full: only the quarters of the tile that have rows
+        if (M - m0 > kBM / 2) body(std::integral_constant<int, MT>{});
+        else if (M - m0 > kBM / 4) body(std::integral_constant<int, MT / 2>{});
+        else body(std::integral_constant<int, MT / 4>{});
     }
 }
 
 // The tile of each GemmTile: 16-row tiles, strips per wavefront, wavefronts.
-template <int BITS, int TILE>
+template <int BITS, int BS, int TILE>
 struct DirectTile {
     static constexpr int MT = TILE == kTile64x128 ? 4 : 8;
-    static constexpr int S = TILE == kTile128x192 && BITS == 4 ? 3 : 2;
+    static constexpr int S = TILE == kTile128x192 && BITS == 4 && BS == 32 ? 3 : 2;
     static constexpr int NW = TILE == kTile128x256 ? 8 : 4;
 };
 
@@ -404,9 +520,9 @@ template <int BITS, int BS, bool HAS_ZP, int TILE, bool NATIVE>
 hipError_t direct_go(const GemmConfig& c, const void* a, const uint8_t* b, const void* s,
                      const uint8_t* z, void* y, int64_t m, int64_t n, int64_t k, float* part,
                      hipStream_t st) {
-    using T = DirectTile<BITS, TILE>;
+    using T = DirectTile<BITS, BS, TILE>;
     if (c.bm != 16 * T::MT || c.bn != 16 * T::S * T::NW) return hipErrorInvalidValue;
-    auto kern = gemm_direct<BITS, BS, HAS_ZP, T::MT, T::S, T::NW, NATIVE>;
+    auto kern = gemm_direct<BITS, BS, HAS_ZP, T::MT, T::S, T::NW, NATIVE, kDense>;
     constexpr int lds = 2 * 16 * T::MT * 256;
     const int ks = part ? c.ksplit : 1;
     const int64_t items = c.tiles_m * c.tiles_n * ks;
@@ -414,7 +530,7 @@ hipError_t direct_go(const GemmConfig& c, const void* a, const uint8_t* b, const
     hipLaunchKernelGGL(kern, grid, dim3(64 * T::NW), lds, st, static_cast<const f16*>(a), b,
                        static_cast<const f16*>(s), z, static_cast<f16*>(y), (int)m, (int)n,
                        (int)k, (int)c.tiles_m, (int)c.tiles_n, ks, ks > 1 ? part : nullptr,
-                       (uint32_t)(m * k * 2));
+                       (uint32_t)(m * k * 2), DirectGroups{});
     if (ks > 1) return launch_splitk_sum(part, y, m * n, ks, st);
     return hipGetLastError();
 }

@@ -82,8 +82,8 @@ hipError_t launch_gemv_stream_cfg(const StreamConfig& c, const void* a, const ui
                                   int64_t k, int bits, int bs, hipStream_t stream);
 
 // Tile shapes of the prefill GEMM: blocks of 32 and more (mnb_gemm_direct.hpp) in rows x columns
-// of a workgroup -- kTile128x192 is 128 x 128 for 8-bit weights, whose operands take twice the
-// registers -- and blocks of 16 (mnb_gemm.hip).
+// of a workgroup -- kTile128x192 is 128 x 128 for all but int4 blocks of 32, whose operands fit the
+// registers with three strips -- and blocks of 16 (mnb_gemm.hip).
 enum GemmTile : int { kTile128x256 = 0, kTile128x192 = 1, kTile64x128 = 2, kTile256x128 = 3 };
 struct GemmConfig {
     int tile;            // GemmTile
@@ -184,6 +184,18 @@ struct StripSwiglu {
     int32_t* pos_of;            // [R], written
     int R, k;
 };
+// The expert-grouped prefill GEMM (mnb_gemm_grouped.hip): Y rows offsets[e] .. offsets[e + 1] - 1
+// = A[row_index[r]] (A[r] without an index) times expert e's int4 weights [n][k / 2], symmetric
+// (zero point 8), scales [n][k / bs]; A has a_rows rows.  b_strips: the experts' MFMA-native strip
+// copies, read in place of b when not null.  swiglu (bias, alpha, beta, limit only) stores the
+// activation instead of Y, row stride n / 2.
+bool gemm_grouped_supported(int64_t rows, int64_t a_rows, int64_t experts, int64_t n, int64_t k,
+                            int bs, const void* a, const void* b);
+hipError_t launch_gemm_grouped(const void* a, int64_t a_rows, const int32_t* row_index,
+                               const int32_t* offsets, int64_t experts, const uint8_t* b,
+                               const uint8_t* b_strips, const void* s, void* y, int64_t rows,
+                               int64_t n, int64_t k, int bs, hipStream_t stream,
+                               const StripSwiglu* swiglu = nullptr);
 // fp16 scales and Y; A is fp16, or for i8 (accuracy_level = 4) the int8 codes of
 // quantize_a_int8 in its quad-interleaved layout (quads = true) with their fp32 scales
 // block-major over 16 rows, a_scale [K / bs][16].

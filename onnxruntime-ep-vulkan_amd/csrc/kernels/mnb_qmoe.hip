@@ -456,6 +456,15 @@ hipError_t launch_qmoe(const QmoeArgs& q, const void* x, const void* logits, con
                        strip_gemv_aligned(x, fc1, fc1_s, nullptr, false) &&
                        strip_geometry(2 * q.inter, q.hidden, q.experts, q.rows, false,
                                       q.block_size, false, &sg);
+    // More expected rows than the strip GEMV's tile: the expert-grouped prefill GEMM (SwiGLU in its
+    // stores for interleaved pairs).  Against the row-tiled GEMV, 2880 x 2880, 32 experts, 4 each:
+    // 72 tokens 154 against 287 us, 256 tokens 198 / 711, 1024 tokens 430 / 1900; 8 experts of
+    // 2048 x 1024, 2 each: 72 tokens 34 / 56, 1024 tokens 81 / 268.
+    const bool tiled = hint > 16 && !strip_gemv_forced_off() &&
+                       gemm_grouped_supported(R, q.rows, q.experts, 2 * q.inter, q.hidden,
+                                              q.block_size, x, fc1) &&
+                       gemm_grouped_supported(R, R, q.experts, q.hidden, q.inter, q.block_size,
+                                              act, fc2);
     const bool self_sort = fused && R <= kSmallR && q.experts <= 64;
     if (self_sort) {
         // sorted inside fc1
@@ -480,8 +489,16 @@ hipError_t launch_qmoe(const QmoeArgs& q, const void* x, const void* logits, con
         e = launch_strip_gemv(sg, false, x, nullptr, row_token, offsets, fc1, fc1_s, nullptr, act,
                               R, 2 * q.inter, q.hidden, q.block_size, st, &sw, fc1_strips);
         if (e != hipSuccess) return e;
+    } else if (tiled && q.fusion == 1) {
+        const StripSwiglu sw{fc1_b, q.alpha, q.beta, q.limit, q.has_limit, nullptr, nullptr,
+                             nullptr, 0, 0};
+        e = launch_gemm_grouped(x, q.rows, row_token, offsets, q.experts, fc1, fc1_strips, fc1_s,
+                                act, R, 2 * q.inter, q.hidden, q.block_size, st, &sw);
+        if (e != hipSuccess) return e;
     } else {
-        e = launch_group_gemv_f16_bounded(x, row_token, offsets, q.experts, q.rows, hint, fc1,
+        e = tiled ? launch_gemm_grouped(x, q.rows, row_token, offsets, q.experts, fc1, fc1_strips,
+                                        fc1_s, h, R, 2 * q.inter, q.hidden, q.block_size, st)
+                  : launch_group_gemv_f16_bounded(x, row_token, offsets, q.experts, q.rows, hint, fc1,
                                           fc1_s, nullptr, h, R, 2 * q.inter, q.hidden, 4,
                                           q.block_size, st);
         if (e != hipSuccess) return e;
@@ -491,9 +508,11 @@ hipError_t launch_qmoe(const QmoeArgs& q, const void* x, const void* logits, con
         e = hipGetLastError();
         if (e != hipSuccess) return e;
     }
-    e = launch_group_gemv_f16_bounded(act, nullptr, offsets, q.experts, q.rows, hint, fc2, fc2_s,
-                                      nullptr, o, R, q.hidden, q.inter, 4, q.block_size, st,
-                                      fc2_strips);
+    e = tiled ? launch_gemm_grouped(act, R, nullptr, offsets, q.experts, fc2, fc2_strips, fc2_s, o,
+                                    R, q.hidden, q.inter, q.block_size, st)
+              : launch_group_gemv_f16_bounded(act, nullptr, offsets, q.experts, q.rows, hint, fc2,
+                                              fc2_s, nullptr, o, R, q.hidden, q.inter, 4,
+                                              q.block_size, st, fc2_strips);
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(qmoe_combine, dim3(grid_for(q.rows * (q.hidden / 8))), dim3(256), 0, st, o,
                        static_cast<const f16*>(fc2_b), expert_of, weight_of, pos_of,

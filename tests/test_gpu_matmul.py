@@ -329,9 +329,10 @@ DIRECT_SHAPES = [
     (127, 129, 448, 4, 64, True, (64, 128)),
     (70, 250, 640, 4, 128, True, (64, 128)),
     (91, 77, 704, 8, 64, True, (64, 128)),
-    (2001, 3050, 320, 4, 64, True, (128, 192)),
+    (2001, 3050, 320, 4, 32, False, (128, 192)),
     (2001, 3050, 384, 4, 32, True, (128, 192)),
-    (1999, 3041, 256, 4, 128, False, (128, 192)),
+    (2040, 6101, 320, 4, 64, True, (128, 128)),
+    (2040, 6100, 256, 4, 128, False, (128, 128)),
     (2040, 8100, 192, 4, 32, True, (128, 256)),
     (2040, 8101, 192, 4, 64, False, (128, 256)),
     (2040, 8100, 128, 4, 128, True, (128, 256)),

@@ -131,6 +131,37 @@ def test_qmoe_skewed_routing_spans_several_row_tiles(cuda):
     _check(y.float().cpu().numpy(), ref16, ref)
 
 
+# Expert row counts around the edges of the grouped GEMM's row tiles (64 rows of a wavefront, 128
+# of a workgroup), experts without rows, and experts past the 64 that one scan of the offsets
+# covers; N = 2I and H are no whole number of column tiles.
+TILE_COUNTS = [0, 1, 63, 64, 65, 127, 128, 129, 200]
+SPARSE_COUNTS = [300 if e in (0, 63, 64, 129) else 0 for e in range(130)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("counts,H,I,bs,fusion,bias", [
+    (TILE_COUNTS, 320, 192, 32, 1, True),
+    (TILE_COUNTS, 320, 192, 64, 2, True),
+    (TILE_COUNTS, 384, 128, 128, 1, False),
+    (SPARSE_COUNTS, 128, 64, 32, 1, True),
+], ids=["bs32", "bs64-concat", "bs128", "sparse"])
+def test_qmoe_grouped_gemm_tile_edges(cuda, counts, H, I, bs, fusion, bias):
+    import mnb
+    import torch
+
+    E, T = len(counts), sum(counts)
+    inp = oq.make_qmoe_inputs(T, H, I, E, block_size=bs, bias=bias, seed=77)
+    owner = np.random.default_rng(78).permutation(np.repeat(np.arange(E), counts))
+    inp["logits"][np.arange(T), owner] = 20.0            # k = 1: exactly `counts` rows each
+    ref16, ref = _refs(inp, 1, I, bs, fusion, 7.0, True)
+    d = {key: _t(v, cuda) for key, v in inp.items()}
+    y = mnb.qmoe(d["x"], d["logits"], d["fc1"], d["fc1_scales"], d["fc2"], d["fc2_scales"], k=1,
+                 inter=I, block_size=bs, fc1_bias=d["fc1_bias"], fc2_bias=d["fc2_bias"],
+                 fusion=fusion, normalize=True, limit=7.0)
+    torch.cuda.synchronize()
+    _check(y.float().cpu().numpy(), ref16, ref)
+
+
 @pytest.mark.gpu
 def test_qmoe_is_deterministic(cuda):
     import mnb
