@@ -591,6 +591,45 @@ static hipError_t gemm_zp(const GemmConfig& c, const void* a, const uint8_t* b, 
     return gemm_go<BITS, BS, false>(c, a, b, s, z, y, m, n, k, part, st);
 }
 
+// ---- 17 to 64 rows ----
+
+bool rows64_geometry(int64_t m, int64_t n, int64_t k, int bits, int bs, Rows64Geom* out) {
+    if (m < 17 || m > 64 || n < 1 || bits != 4 || (bs != 32 && bs != 64 && bs != 128)) return false;
+    if (!gemm_supported(m, n, k, bits, bs, false)) return false;
+    Rows64Geom g{};
+    g.mt = (int)((m + 15) / 16);
+    // Strips per workgroup: the fewest cycles of a CU, rounds of (the copy of A at 64 bytes per
+    // clock + per strip and 32-k chunk 4 mt rescale FMAs and about 13 unpack instructions on a
+    // quarter of the chip's SIMD lanes).
+    const int64_t strips = (n + 15) / 16;
+    int64_t best = 0;
+    for (int s = 1; s <= 4; ++s) {
+        const int64_t gx = (strips + s - 1) / s;
+        const int64_t cycles = ((gx + 255) / 256) *
+                               (g.mt * 16 * k * 2 / 64 + s * (k / 32) * (4 * g.mt + 13));
+        if (best == 0 || cycles < best) {
+            best = cycles;
+            g.s = s;
+            g.gx = gx;
+        }
+    }
+    // eight wavefronts' two 64-k stages of A, or their partial tiles
+    g.lds = (size_t)8 * g.mt * std::max(2 * 2048, g.s * 1024);
+    *out = g;
+    return true;
+}
+
+hipError_t launch_rows64(const Rows64Geom& g, const void* a, const uint8_t* b, const void* s,
+                         const uint8_t* z, void* y, int64_t m, int64_t n, int64_t k, int bs,
+                         hipStream_t st, const uint8_t* b_strips) {
+    switch (bs) {
+        case 32: return launch_rows64_bs32(g, a, b, b_strips, s, z, y, m, n, k, st);
+        case 64: return launch_rows64_bs64(g, a, b, b_strips, s, z, y, m, n, k, st);
+        case 128: return launch_rows64_bs128(g, a, b, b_strips, s, z, y, m, n, k, st);
+        default: return hipErrorInvalidValue;
+    }
+}
+
 hipError_t launch_gemm(const void* a, const uint8_t* b, const void* s, const uint8_t* z, void* y,
                        int64_t m, int64_t n, int64_t k, int bits, int bs, hipStream_t st,
                        void* workspace, size_t workspace_bytes, const uint8_t* b_strips) {

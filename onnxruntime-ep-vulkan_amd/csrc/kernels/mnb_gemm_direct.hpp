@@ -126,6 +126,86 @@ __device__ __forceinline__ T load_any(const void* p) {
     return v;
 }
 
+// Block scales and zero points of a pair of quads (from an even one) for S strips: a column's
+// 2 BPQ scales and zero points are consecutive bytes, read by one load each (scattered loads cost
+// the wavefront far more than their bytes).  A pair that runs past the column's end is read block
+// by block.
+template <int BITS, int BS, bool HAS_ZP, int S>
+struct ScalePair {
+    static constexpr int NSC = 2 * 128 / BS;             // 8, 4 or 2 blocks
+    uint32_t sc[S][NSC / 2];
+    uint32_t z[S][BITS == 8 ? 2 : 1];
+
+    // s_off, z_off: byte offset of each strip's column; b: the pair's first block
+    __device__ __forceinline__ void load(const f16* Sc, const uint8_t* Z, const uint32_t (&s_off)[S],
+                                         const uint32_t (&z_off)[S], int b, int bpc, int zpb) {
+        if (b + NSC <= bpc) {
+#pragma unroll
+            for (int t = 0; t < S; ++t) {
+                const uint8_t* sp = reinterpret_cast<const uint8_t*>(Sc) + (int64_t)b * 2 + s_off[t];
+                if constexpr (NSC == 8) {
+                    const u32x4 v = load_any<u32x4>(sp);
+                    sc[t][0] = v.x;
+                    sc[t][1] = v.y;
+                    sc[t][NSC / 2 - 2] = v.z;
+                    sc[t][NSC / 2 - 1] = v.w;
+                } else if constexpr (NSC == 4) {
+                    const u32x2 v = load_any<u32x2>(sp);
+                    sc[t][0] = v.x;
+                    sc[t][1] = v.y;
+                } else {
+                    sc[t][0] = load_any<uint32_t>(sp);
+                }
+                if constexpr (HAS_ZP) {
+                    const uint8_t* zp = Z + (BITS == 8 ? b : b >> 1) + z_off[t];
+                    constexpr int ZB = NSC * BITS / 8;   // 1 to 8 bytes
+                    if constexpr (ZB == 8) {
+                        const u32x2 v = load_any<u32x2>(zp);
+                        z[t][0] = v.x;
+                        z[t][BITS == 8] = v.y;
+                    } else if constexpr (ZB == 4) {
+                        z[t][0] = load_any<uint32_t>(zp);
+                    } else if constexpr (ZB == 2) {
+                        z[t][0] = load_any<uint16_t>(zp);
+                    } else {
+                        z[t][0] = *zp;
+                    }
+                }
+            }
+        } else {
+#pragma unroll
+            for (int t = 0; t < S; ++t) {
+                const uint16_t* sp = reinterpret_cast<const uint16_t*>(
+                    reinterpret_cast<const uint8_t*>(Sc) + s_off[t]);
+#pragma unroll
+                for (uint32_t& v : z[t]) v = 0;
+#pragma unroll
+                for (int i = 0; i < NSC; i += 2) {
+                    sc[t][i / 2] = sp[min(b + i, bpc - 1)] |
+                                   ((uint32_t)sp[min(b + i + 1, bpc - 1)] << 16);
+                    if constexpr (HAS_ZP && BITS == 8) {
+                        z[t][i / 4] |= ((uint32_t)Z[z_off[t] + min(b + i, zpb - 1)] |
+                                        (uint32_t)Z[z_off[t] + min(b + i + 1, zpb - 1)] << 8)
+                                       << (8 * (i & 3));
+                    } else if constexpr (HAS_ZP) {
+                        z[t][0] |= (uint32_t)Z[z_off[t] + min((b + i) >> 1, zpb - 1)] << (4 * i);
+                    }
+                }
+            }
+        }
+    }
+    // scale and zero point of block bi of the pair (a compile-time constant)
+    __device__ __forceinline__ float scale(int t, int bi) const {
+        const uint32_t w = sc[t][bi >> 1];
+        return (float)__builtin_bit_cast(f16, (uint16_t)(bi & 1 ? w >> 16 : w & 0xFFFFu));
+    }
+    __device__ __forceinline__ uint32_t zero(int t, int bi) const {
+        if constexpr (!HAS_ZP) return 1u << (BITS - 1);
+        return __builtin_amdgcn_ubfe(z[t][BITS == 8 ? bi >> 2 : 0],
+                                     BITS == 8 ? 8 * (bi & 3) : 4 * bi, BITS);
+    }
+};
+
 }  // namespace
 
 // MT: 16-row tiles per workgroup; S: 16-column strips per wavefront; NW: wavefronts per workgroup,
@@ -229,71 +309,7 @@ gemm_direct(const f16* __restrict__ A, const uint8_t* __restrict__ B, const f16*
 #pragma unroll
             for (int h = 0; h < WPL; ++h) w[t][h] = buffer_load16(rb, b_off[t] + 16 * h, (uint32_t)so);
     };
-    // Block scales and zero points of a pair of quads: 2 BPQ scales and nibbles of a column are
-    // consecutive bytes, read by one load each (scattered loads cost the wavefront far more than
-    // their bytes).  A pair that runs past the column's end is read block by block.
-    constexpr int NSC = 2 * BPQ;                         // 8, 4 or 2 blocks
-    struct Pair {
-        uint32_t sc[S][NSC / 2];
-        uint32_t z[S][BITS == 8 ? 2 : 1];
-    };
-    auto load_p = [&](Pair& r, int q) {
-        const int b = q * BPQ;
-        if (b + NSC <= bpc) {
-#pragma unroll
-            for (int t = 0; t < S; ++t) {
-                const uint8_t* sp = reinterpret_cast<const uint8_t*>(Sc) + (int64_t)b * 2 + s_off[t];
-                if constexpr (NSC == 8) {
-                    const u32x4 v = load_any<u32x4>(sp);
-                    r.sc[t][0] = v.x;
-                    r.sc[t][1] = v.y;
-                    r.sc[t][2] = v.z;
-                    r.sc[t][3] = v.w;
-                } else if constexpr (NSC == 4) {
-                    const u32x2 v = load_any<u32x2>(sp);
-                    r.sc[t][0] = v.x;
-                    r.sc[t][1] = v.y;
-                } else {
-                    r.sc[t][0] = load_any<uint32_t>(sp);
-                }
-                if constexpr (HAS_ZP) {
-                    const uint8_t* zp = Z + (BITS == 8 ? b : b >> 1) + z_off[t];
-                    constexpr int ZB = NSC * BITS / 8;   // 1 to 8 bytes
-                    if constexpr (ZB == 8) {
-                        const u32x2 v = load_any<u32x2>(zp);
-                        r.z[t][0] = v.x;
-                        r.z[t][BITS == 8] = v.y;
-                    } else if constexpr (ZB == 4) {
-                        r.z[t][0] = load_any<uint32_t>(zp);
-                    } else if constexpr (ZB == 2) {
-                        r.z[t][0] = load_any<uint16_t>(zp);
-                    } else {
-                        r.z[t][0] = *zp;
-                    }
-                }
-            }
-        } else {
-#pragma unroll
-            for (int t = 0; t < S; ++t) {
-                const uint16_t* sp = reinterpret_cast<const uint16_t*>(
-                    reinterpret_cast<const uint8_t*>(Sc) + s_off[t]);
-#pragma unroll
-                for (uint32_t& z : r.z[t]) z = 0;
-#pragma unroll
-                for (int i = 0; i < NSC; i += 2) {
-                    r.sc[t][i / 2] = sp[min(b + i, bpc - 1)] |
-                                     ((uint32_t)sp[min(b + i + 1, bpc - 1)] << 16);
-                    if constexpr (HAS_ZP && BITS == 8) {
-                        r.z[t][i / 4] |= ((uint32_t)Z[z_off[t] + min(b + i, zpb - 1)] |
-                                          (uint32_t)Z[z_off[t] + min(b + i + 1, zpb - 1)] << 8)
-                                         << (8 * (i & 3));
-                    } else if constexpr (HAS_ZP) {
-                        r.z[t][0] |= (uint32_t)Z[z_off[t] + min((b + i) >> 1, zpb - 1)] << (4 * i);
-                    }
-                }
-            }
-        }
-    };
+    using Pair = ScalePair<BITS, BS, HAS_ZP, S>;
 
     // The K loop and the stores over the first MV row tiles.
     auto body = [&](auto mt_c) {
@@ -366,13 +382,9 @@ gemm_direct(const f16* __restrict__ A, const uint8_t* __restrict__ B, const f16*
 #pragma unroll
                 for (int t = 0; t < S; ++t) {
                     const int bi = half * BPQ + bq;          // block of the pair
-                    const uint32_t sw = r.sc[t][bi >> 1];
-                    sc[t] = (float)__builtin_bit_cast(f16, (uint16_t)(bi & 1 ? sw >> 16 : sw & 0xFFFFu));
+                    sc[t] = r.scale(t, bi);
                     asm volatile("" : "+v"(sc[t]));
-                    uint32_t z = 1u << (BITS - 1);
-                    if constexpr (HAS_ZP)
-                        z = __builtin_amdgcn_ubfe(r.z[t][BITS == 8 ? bi >> 2 : 0],
-                                                  BITS == 8 ? 8 * (bi & 3) : 4 * bi, BITS);
+                    const uint32_t z = r.zero(t, bi);
 #pragma unroll
                     for (int cc = 0; cc < CPB; ++cc) {
                         const uint32_t w = wv[t][0][bq * CPB + cc];
@@ -426,7 +438,7 @@ gemm_direct(const f16* __restrict__ A, const uint8_t* __restrict__ B, const f16*
                 issue_a(q + 1, 16 * MV);
                 load_w(next, q + 1);
                 if constexpr (decltype(half)::value == 0) {
-                    if (q + 2 < q1) load_p(pn, q + 2);
+                    if (q + 2 < q1) pn.load(Sc, Z, s_off, z_off, (q + 2) * BPQ, bpc, zpb);
                 }
             }
             __builtin_amdgcn_sched_barrier(0);
@@ -436,7 +448,7 @@ gemm_direct(const f16* __restrict__ A, const uint8_t* __restrict__ B, const f16*
         using H1 = std::integral_constant<int, 1>;
         issue_a(q0, 16 * MV);
         load_w(w0, q0);
-        load_p(p0, q0);
+        p0.load(Sc, Z, s_off, z_off, q0 * BPQ, bpc, zpb);
         for (int q = q0; q < q1; q += 4) {
             step(q, w0, w1, p0, p1, H0{});
             if (q + 1 >= q1) break;

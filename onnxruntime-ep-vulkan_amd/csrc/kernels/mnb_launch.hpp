@@ -116,6 +116,28 @@ hipError_t launch_gemm_direct_b8(int bs, const GemmConfig& c, const void* a, con
 hipError_t launch_splitk_sum(const float* part, void* y, int64_t mn, int ksplit,
                              hipStream_t stream);
 
+// 17 to 64 fp16 rows, int4, blocks of 32 to 128, K % 64 == 0 (mnb_rows64.hpp): s 16-column strips
+// and all the rows (mt 16-row tiles) per workgroup of eight wavefronts, K split over them.
+struct Rows64Geom {
+    int mt, s;           // 2..4, 1..4
+    int64_t gx;          // workgroups
+    size_t lds;
+};
+bool rows64_geometry(int64_t m, int64_t n, int64_t k, int bits, int bs, Rows64Geom* out);
+// b_strips: the MFMA-native strip copy of B (launch_strip_pack), read in place of b when not null.
+hipError_t launch_rows64(const Rows64Geom& g, const void* a, const uint8_t* b, const void* s,
+                         const uint8_t* z, void* y, int64_t m, int64_t n, int64_t k, int bs,
+                         hipStream_t stream, const uint8_t* b_strips);
+hipError_t launch_rows64_bs32(const Rows64Geom& g, const void* a, const uint8_t* b,
+                              const uint8_t* strips, const void* s, const uint8_t* z, void* y,
+                              int64_t m, int64_t n, int64_t k, hipStream_t stream);
+hipError_t launch_rows64_bs64(const Rows64Geom& g, const void* a, const uint8_t* b,
+                              const uint8_t* strips, const void* s, const uint8_t* z, void* y,
+                              int64_t m, int64_t n, int64_t k, hipStream_t stream);
+hipError_t launch_rows64_bs128(const Rows64Geom& g, const void* a, const uint8_t* b,
+                               const uint8_t* strips, const void* s, const uint8_t* z, void* y,
+                               int64_t m, int64_t n, int64_t k, hipStream_t stream);
+
 // Launch shape of the row-tiled MFMA GEMV (mnb_group_gemv.hip).
 struct GroupGeom {
     int mt;              // 16-row tiles per workgroup (1, 2 or 4)
@@ -314,7 +336,8 @@ struct GqaArgs {
     bool copy_past;      // present is its own buffer: the past tokens are copied into it
 };
 struct GqaPlan {
-    int waves;           // wavefronts per workgroup (16 query rows each)
+    int waves;           // wavefronts per workgroup
+    int qt;              // 16-row query tiles per wavefront
     int splits;          // workgroups along the keys of one row block
     int64_t row_blocks;  // row blocks per (batch, KV head)
     int64_t chunk;       // keys per split (a multiple of 64)

@@ -274,6 +274,14 @@ static int plan_search(const mnb_problem* p, mnb_plan_info* out) {
         out->tile_m = 16;
         out->grid_x = sg.gx;
         out->grid_y = sg.gz;
+    } else if (mnb::Rows64Geom r6{}; kern == MNB_KERNEL_GROUP_MFMA && !forced &&
+               mnb::rows64_geometry(p->m, p->n, p->k, p->bits, p->block_size, &r6)) {
+        // 17 to 64 rows: all of them in one workgroup, K split over its wavefronts
+        out->waves_per_group = 8;
+        out->tile_n = 16 * r6.s;
+        out->tile_m = 16 * r6.mt;
+        out->grid_x = r6.gx;
+        out->grid_y = 1;
     } else if (kern == MNB_KERNEL_GROUP_MFMA) {
         const mnb::GroupGeom g =
             mnb::group_geometry(p->m, p->n, p->k, 1, false, p->block_size, false);
@@ -419,6 +427,11 @@ static int matmul_impl(const mnb_problem* p, const void* a, const uint8_t* b,
             return fail(MNB_ERR_UNSUPPORTED, "strip GEMV geometry");
         e = mnb::launch_strip_gemv(sg, false, a, nullptr, nullptr, nullptr, b, scales, zero_points, y,
                                    p->m, p->n, p->k, p->block_size, st);
+    } else if (mnb::Rows64Geom r6{}; kern == MNB_KERNEL_GROUP_MFMA && forced_kernel() == 0 &&
+               aligned(a, 16) && aligned(b, 16) && aligned(scales, 2) &&
+               mnb::rows64_geometry(p->m, p->n, p->k, p->bits, p->block_size, &r6)) {
+        e = mnb::launch_rows64(r6, a, b, scales, zero_points, y, p->m, p->n, p->k, p->block_size,
+                               st, b_strips);
     } else if (kern == MNB_KERNEL_GROUP_MFMA) {
         e = mnb::launch_group_gemv_f16(a, nullptr, nullptr, 1, p->m, b, scales, zero_points, y,
                                        p->m, p->n, p->k, p->bits, p->block_size, st);

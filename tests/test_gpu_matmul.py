@@ -389,6 +389,61 @@ def test_gemm_direct_tiles(cuda, M, N, K, bits, bs, zp, tile, layout):
     _check_f16(y.cpu().numpy(), ref, f"direct {M}x{N}x{K}")
 
 
+# 17 to 64 rows: every row-tile count at its edges, 1 to 4 strips per workgroup and N off a strip,
+# fewer quads than wavefronts, odd quad counts, a last half quad, K / bs odd.
+ROWS64_SHAPES = [
+    (17, 100, 64, 32, True, 1),
+    (32, 48, 1600, 32, False, 1),
+    (33, 4100, 1152, 64, True, 2),
+    (48, 9216, 1088, 32, True, 3),
+    (49, 8200, 576, 64, True, 3),
+    (64, 16384, 512, 32, False, 4),
+    (64, 16370, 640, 128, True, 4),
+    (47, 3072, 3072, 128, False, 1),
+    (20, 5000, 2880, 64, True, 2),
+]
+
+
+@pytest.mark.parametrize("layout", ["ort", "strips"])
+@pytest.mark.parametrize("M,N,K,bs,zp,strips", ROWS64_SHAPES)
+def test_rows64(cuda, M, N, K, bs, zp, strips, layout):
+    import ctypes as C
+    import mnb
+    import torch
+
+    p = mnb.problem(M, N, K, 4, bs, zp)
+    info = mnb.plan(p)
+    assert (info.kernel, info.tile_m, info.tile_n) == (mnb.KERNEL_GROUP_MFMA, -(-M // 16) * 16,
+                                                       16 * strips)
+    inp = orc.make_inputs(M, N, K, bits=4, block_size=bs, with_zp=zp, seed=M + N + K)
+    t = {k: _dev(v, cuda) for k, v in inp.items() if v is not None}
+    print(f"[gpu] rows64 {M}x{N}x{K} bs={bs} {layout}", flush=True)
+    y = torch.empty(M, N, dtype=torch.float16, device=cuda)
+    if layout == "strips":
+        lib, s, w = mnb.load(), C.c_void_p(), C.c_void_p()
+        mnb.check(lib.mnb_session_create(0, C.byref(s)))
+        z = inp["zp"]
+        mnb.check(lib.mnb_weights_upload(
+            s, C.byref(p), inp["B"].ctypes.data, inp["B"].nbytes, inp["scales"].ctypes.data,
+            inp["scales"].nbytes, z.ctypes.data if zp else None, z.nbytes if zp else 0, C.byref(w)))
+        rc = lib.mnb_weights_prepack(w, None)
+        torch.cuda.synchronize()
+        if rc == mnb.MNB_OK:
+            mnb.check(lib.mnb_session_run(s, w, M, t["A"].data_ptr(), 1, y.data_ptr(), 1))
+        mnb.check(lib.mnb_weights_release(w))
+        mnb.check(lib.mnb_session_destroy(s))
+        if rc == mnb.MNB_ERR_UNSUPPORTED:
+            pytest.skip("the node has no strip copy")
+        mnb.check(rc)
+    else:
+        mnb.matmul_nbits(t["A"], t["B"], t["scales"], t.get("zp"), N, K, 4, bs, out=y)
+    torch.cuda.synchronize()
+    w64 = torch.from_numpy(orc.dequantize_f32(inp["B"], inp["scales"], inp["zp"], N, K, 4, bs)
+                           .astype(np.float64)).to(cuda)
+    ref = (t["A"].double() @ w64.t()).cpu().numpy()
+    _check_f16(y.cpu().numpy(), ref, f"rows64 {M}x{N}x{K}")
+
+
 def test_gemm_uneven_k_split(cuda):
     """K split whose last split is shorter: K = 1600 is 25 steps of 64, over 3 workgroups per tile
     (9, 9 and 7 steps).  Checked against the oracle, and against the same GEMM run unsplit (no
