@@ -44,7 +44,7 @@ def _t(a, dev):
     return torch.from_numpy(np.ascontiguousarray(a)).to(dev)
 
 
-def _check(inp, attn, prk, prv, Nq, Nkv, scale=None):
+def _check(inp, attn, prk, prv, Nq, Nkv, scale=None, significant=2e-3):
     B, S, _ = inp["qkv"].shape
     total = int(inp["past_k"].shape[2]) + S
     want, wk, wv = og.gqa(inp["qkv"], inp["past_k"], inp["past_v"], inp["seqlens_k"], total,
@@ -52,7 +52,7 @@ def _check(inp, attn, prk, prv, Nq, Nkv, scale=None):
                           f16_points=True)
     attn = np.asarray(attn, dtype=np.float64)
     assert np.all(np.isfinite(attn))
-    assert orc.max_rel_err_significant(attn, want) <= 2e-3
+    assert orc.max_rel_err_significant(attn, want) <= significant
     assert orc.max_err_rms_normalised(attn, want) <= 2e-3
     for b in range(B):
         past_len = max(int(inp["seqlens_k"][b]) + 1 - S, 0)
@@ -103,6 +103,58 @@ def test_reference_decode_shape(cuda, past):
 def test_matches_oracle(cuda, B, S, past, Nq, Nkv, D):
     inp = _inputs(B, S, [past + S - 1] * B, Nq, Nkv, D, past_buffer=past, seed=B * 7 + S + past)
     _check(inp, *_run(cuda, inp, Nq, Nkv), Nq, Nkv)
+
+
+@pytest.mark.parametrize("B,S,past,Nq,Nkv,D", [
+    (4, 260, 40, 32, 32, 64),    # two query tiles per wavefront: 128-row blocks, the last of 4 rows
+    (3, 300, 0, 32, 32, 96),     # ... whole heads per XCD
+    (16, 65, 0, 64, 16, 128),    # ... 4 query heads per KV head
+    (5, 129, 3, 64, 32, 112),    # ... a 16-deep tail, workgroups not a multiple of 8
+    (2, 70, 5, 8, 8, 144),       # above 128 dims: one tile per wavefront
+    (1, 4, 4092, 4, 1, 128),     # 16 rows, 64 splits of one 64-key block
+    (2, 2, 63, 8, 2, 96),        # splits that end on a block's edge
+])
+def test_attend_tiles(cuda, B, S, past, Nq, Nkv, D):
+    """The significant-element bar is 4e-3 here: a rotated key within fp32 rounding of a tie is
+    stored as the neighbouring fp16 (2^-10 of it) and moves its score by up to 2^-10 |k_d q_d| scale,
+    about 1e-3 at |k_d|, |q_d| = 3; among the 0.8 to 4.3 million outputs of these cases some small
+    one (0.1 RMS) gets two such moves and its own rounding (2^-11)."""
+    inp = _inputs(B, S, [past + S - 1] * B, Nq, Nkv, D, past_buffer=past, seed=3 * B + S + past)
+    _check(inp, *_run(cuda, inp, Nq, Nkv), Nq, Nkv, significant=4e-3)
+
+
+@pytest.mark.parametrize("scale", [-0.2, 1e-24, 0.0])
+def test_scale_sign_and_vanishing_scale(cuda, scale):
+    inp = _inputs(1, 70, [79], 4, 2, 64, past_buffer=10, seed=16)
+    _check(inp, *_run(cuda, inp, 4, 2, scale=scale), 4, 2, scale=scale)
+
+
+@pytest.mark.parametrize("rd", [4, 20])
+def test_rotary_dims_off_the_chunk(cuda, rd):
+    """Half rotary widths that are no multiple of 8 take the element-wise rotation."""
+    inp = _inputs(2, 9, [20, 12], 8, 2, 32, past_buffer=12, rotary_dim=rd, seed=rd)
+    _check(inp, *_run(cuda, inp, 8, 2), 8, 2)
+
+
+@pytest.mark.parametrize("S,seqlens", [(5, [30, 33]), (20, [31, 40])])
+def test_new_tokens_past_the_end_of_a_shared_buffer(cuda, S, seqlens):
+    """A shared buffer of 32 positions that does not hold all of a batch row's new tokens: they
+    attend to their own keys all the same, as the same call with a growing cache does."""
+    import mnb
+    import torch
+
+    inp = _inputs(2, S, seqlens, 8, 2, 64, past_buffer=32, seed=S)
+    grown, gk, gv = _run(cuda, inp, 8, 2)
+    d = {k: _t(inp[k], cuda) for k in ("qkv", "past_k", "past_v", "seqlens_k", "cos", "sin")}
+    attn, k, v = mnb.gqa(d["qkv"], d["past_k"], d["past_v"], d["seqlens_k"], d["cos"], d["sin"],
+                         num_heads=8, kv_num_heads=2, rotary_dim=inp["rd"], present_k=d["past_k"],
+                         present_v=d["past_v"])
+    torch.cuda.synchronize()
+    assert orc.max_err_rms_normalised(attn.cpu().numpy(), grown.astype(np.float64)) <= 1e-3
+    for b in range(2):                                   # the positions that exist hold the same
+        hi = min(32, max(seqlens[b] + 1 - S, 0) + S)
+        assert np.array_equal(k.cpu().numpy()[b, :, :hi], gk[b, :, :hi])
+        assert np.array_equal(v.cpu().numpy()[b, :, :hi], gv[b, :, :hi])
 
 
 def test_ragged_batch_and_partial_rotary(cuda):
