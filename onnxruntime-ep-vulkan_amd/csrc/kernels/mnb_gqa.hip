@@ -78,6 +78,18 @@ __device__ __forceinline__ bool new_in_present(int64_t past_len, const GqaDims& 
     return past_len + g.S <= g.present_len;
 }
 
+// Buffer descriptor over `bytes` bytes at a wave-uniform address (loads past them return zero).
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const f16* p, uint32_t bytes) {
+    const uint64_t a = reinterpret_cast<uint64_t>(p);
+    const uint64_t u = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a) |
+                       (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32;
+    return __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<void*>(u), 0,
+                                             __builtin_amdgcn_readfirstlane((int)bytes), 0x00027000);
+}
+__device__ __forceinline__ u32x4 buffer_load16(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff) {
+    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, (int)soff, 0));
+}
+
 // LDS row of key kk within a 64-key block: the 16 keys one score MFMA reads (see gqa_attend)
 // sit in 16 consecutive rows.
 __device__ __forceinline__ int lds_row(int kk) {
@@ -290,34 +302,30 @@ gqa_attend(const f16* __restrict__ qr, const f16* __restrict__ past_k,
     u32x4 kreg[KIT];
     u32x4 vreg[VIT][4];
 
+    // Blocks of up to 64 keys, none across past_len (the keys' source changes there): block
+    // [kb, block_end(kb)).
+    auto block_end = [&](int64_t kb) {
+        const int64_t stop = kb < past_len ? std::min(past_len, k_stop) : k_stop;
+        return std::min<int64_t>(kb + kBN, stop);
+    };
+    // One block into registers.  K: 16 bytes per item, items of a key consecutive; V: 8 dims of 4
+    // keys per item.  Buffer loads from the block's own (uniform) base, whose bound makes keys past
+    // its end zeros.  (Picking source and bound per lane put every load behind a branch of its
+    // own, and the wait for each cost 2,600 of a block's 8,400 cycles.)
     auto load = [&](int64_t kb) {
+        const bool in_past = kb < past_len;
+        const uint32_t bytes = (uint32_t)(block_end(kb) - kb) * (D * 2);
+        const auto rk = buffer_of((in_past ? pk_base : kn_base) + kb * D, bytes);
+        const auto rv = buffer_of((in_past ? pv_base : vn_base) + kb * D, bytes);
 #pragma unroll
-        for (int it = 0; it < KIT; ++it) {
-            const int c = tid + NT * it;
-            if (c < KCH) {
-                const int64_t t = kb + c / CPR;
-                const int part = c % CPR;
-                kreg[it] = u32x4{0, 0, 0, 0};
-                if (t < k_stop)
-                    kreg[it] = *reinterpret_cast<const u32x4*>(
-                        (t < past_len ? pk_base : kn_base) + t * D + 8 * part);
-            }
-        }
+        for (int it = 0; it < KIT; ++it) kreg[it] = buffer_load16(rk, (uint32_t)(tid + NT * it) * 16, 0);
 #pragma unroll
         for (int it = 0; it < VIT; ++it) {
             const int c = tid + NT * it;
-            if (c < VITEMS) {
-                const int kg = c & 15;
-                const int dc = c >> 4;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const int64_t t = kb + 4 * kg + q;
-                    vreg[it][q] = u32x4{0, 0, 0, 0};
-                    if (t < k_stop)
-                        vreg[it][q] = *reinterpret_cast<const u32x4*>(
-                            (t < past_len ? pv_base : vn_base) + t * D + 8 * dc);
-                }
-            }
+            for (int q = 0; q < 4; ++q)
+                vreg[it][q] = buffer_load16(
+                    rv, (uint32_t)((4 * (c & 15) + q) * D + 8 * (c >> 4)) * 2, 0);
         }
     };
 
@@ -325,19 +333,15 @@ gqa_attend(const f16* __restrict__ qr, const f16* __restrict__ past_k,
 #pragma unroll
         for (int it = 0; it < KIT; ++it) {
             const int c = tid + NT * it;
-            if (c < KCH) {
+            if (KCH % NT == 0 || c < KCH) {
                 const int kk = c / CPR;
-                const int part = c % CPR;
-                *reinterpret_cast<u32x4*>(&Ks[lds_row(kk) * KP + 8 * part]) = kreg[it];
-                const int64_t t = kb + kk;
-                if (copy && t < past_len)
-                    *reinterpret_cast<u32x4*>(prk + t * D + 8 * part) = kreg[it];
+                *reinterpret_cast<u32x4*>(&Ks[lds_row(kk) * KP + 8 * (c % CPR)]) = kreg[it];
             }
         }
 #pragma unroll
         for (int it = 0; it < VIT; ++it) {
             const int c = tid + NT * it;
-            if (c < VITEMS) {
+            if (VITEMS % NT == 0 || c < VITEMS) {
                 const int kg = c & 15;
                 const int dc = c >> 4;
                 const f16x8 v0 = __builtin_bit_cast(f16x8, vreg[it][0]);
@@ -349,19 +353,32 @@ gqa_attend(const f16* __restrict__ qr, const f16* __restrict__ past_k,
                     const h4 col = {v0[e], v1[e], v2[e], v3[e]};
                     *reinterpret_cast<h4*>(&Vt[(8 * dc + e) * kVP + 4 * kg]) = col;
                 }
-                if (copy) {
+            }
+        }
+        if (copy && kb < past_len) {                     // uniform: past tokens into present
+            const int64_t kend = block_end(kb);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const int64_t t = kb + 4 * kg + q;
-                        if (t < past_len)
-                            *reinterpret_cast<u32x4*>(prv + t * D + 8 * dc) = vreg[it][q];
-                    }
+            for (int it = 0; it < KIT; ++it) {
+                const int c = tid + NT * it;
+                const int64_t t = kb + c / CPR;
+                if (c < KCH && t < kend)
+                    *reinterpret_cast<u32x4*>(prk + t * D + 8 * (c % CPR)) = kreg[it];
+            }
+#pragma unroll
+            for (int it = 0; it < VIT; ++it) {
+                const int c = tid + NT * it;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int64_t t = kb + 4 * (c & 15) + q;
+                    if (c < VITEMS && t < kend)
+                        *reinterpret_cast<u32x4*>(prv + t * D + 8 * (c >> 4)) = vreg[it][q];
                 }
             }
         }
     };
 
     auto compute = [&](int64_t kb) {
+        const int64_t kend = block_end(kb);
         // S^T tiles: c2 = 32-key half, a = 16-key MFMA tile.  Lane (j, grp) ends up with the
         // scores of query j and keys kb + 32 c2 + 8 grp + 4 a + i.
         f32x4 sc[QT][2][2];
@@ -396,14 +413,17 @@ gqa_attend(const f16* __restrict__ qr, const f16* __restrict__ past_k,
         f16x8 pb[QT][2], pl[QT][2];                      // P = pb + pl to 2^-22
 #pragma unroll
         for (int u = 0; u < QT; ++u) {
-            if (kb + kBN - 1 > tp_lo[u]) {               // uniform: the block crosses the diagonal
+            // uniform: the block crosses the diagonal, or is short
+            if (kb + kBN - 1 > tp_lo[u] || kend - kb < kBN) {
+                // first masked key of the lane, counted from its first key of the block
+                const int cut = (int)std::min<int64_t>(tp[u] + 1 - kb, kend - kb) - 8 * grp;
 #pragma unroll
                 for (int c2 = 0; c2 < 2; ++c2)
 #pragma unroll
                     for (int a = 0; a < 2; ++a)
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
-                            if (kb + 32 * c2 + 8 * grp + 4 * a + i > tp[u]) sc[u][c2][a][i] = -INFINITY;
+                            if (32 * c2 + 4 * a + i >= cut) sc[u][c2][a][i] = -INFINITY;
             }
             float mloc = -INFINITY;
 #pragma unroll
@@ -428,16 +448,20 @@ gqa_attend(const f16* __restrict__ qr, const f16* __restrict__ past_k,
 #pragma unroll
             for (int c2 = 0; c2 < 2; ++c2)
 #pragma unroll
-                for (int a = 0; a < 2; ++a)
+                for (int i = 0; i < 8; i += 2) {
+                    float p[2];
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const float p = __builtin_amdgcn_exp2f(
-                            __builtin_fmaf(sc[u][c2][a][i], g.scale_log2, -m_new));
-                        l += p;
-                        const f16 hi = (f16)p;
-                        pb[u][c2][4 * a + i] = hi;
-                        pl[u][c2][4 * a + i] = (f16)(p - (float)hi);
+                    for (int e = 0; e < 2; ++e) {
+                        p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(
+                            sc[u][c2][i >> 2][(i & 3) + e], g.scale_log2, -m_new));
+                        l += p[e];
                     }
+                    const f16x2 hi = {(f16)p[0], (f16)p[1]};
+                    pb[u][c2][i] = hi.x;
+                    pb[u][c2][i + 1] = hi.y;
+                    pl[u][c2][i] = (f16)__builtin_fmaf((float)hi.x, -1.f, p[0]);
+                    pl[u][c2][i + 1] = (f16)__builtin_fmaf((float)hi.y, -1.f, p[1]);
+                }
             l_run[u] += l;
         }
         // O^T += V^T P^T over keys kb + 32 c2 + 8 grp .. + 7.
@@ -456,15 +480,15 @@ gqa_attend(const f16* __restrict__ qr, const f16* __restrict__ past_k,
             }
     };
 
-    const int64_t nblk = (k_stop - k_begin + kBN - 1) / kBN;
     load(k_begin);
-    for (int64_t ib = 0; ib < nblk; ++ib) {
-        const int64_t kb = k_begin + ib * kBN;
-        if (ib) __syncthreads();                         // the previous block is consumed
+    for (int64_t kb = k_begin; kb < k_stop;) {
+        const int64_t next = block_end(kb);
+        if (kb != k_begin) __syncthreads();              // the previous block is consumed
         store(kb);
         __syncthreads();
-        if (ib + 1 < nblk) load(kb + kBN);
+        if (next < k_stop) load(next);
         if (wave_active && kb <= tp_hi) compute(kb);
+        kb = next;
     }
 
 #pragma unroll
