@@ -25,7 +25,7 @@
 //                r = s * G + g) as fp16 high and low parts, and the present writes.  Bound by its
 //                bytes (S = 2048, 32 + 64 heads of 96: 88 MB); one dim per thread and 64-bit
 //                divisions took 80 us there, and new K and V also went to the workspace.
-//   gqa_attend   flash attention on v_mfma_f32_16x16x32_f16.  A workgroup takes 16 QT x W query
+//   gqa_attend   flash attention on v_mfma_f32_16x16x32_f16.  A workgroup takes 16 x W query
 //                rows of one (batch, KV head) and walks 64-key blocks staged in LDS (K row-major,
 //                V transposed), the next block in flight in registers.  Scores are computed
 //                transposed, S^T = K Q^T, so each lane holds one query's 16 scores of a block:
@@ -35,11 +35,12 @@
 //                enter the MFMAs as fp16 high + low pairs (two MFMAs each), so scores and weights
 //                keep fp32 precision as in the reference's fp32 kernel; rounding either to one
 //                fp16 costs up to 6e-3 relative on outputs.
-//                Long prompts (QT = 2) are bound by the matrix cores and the softmax's VALU work
-//                about equally; two query tiles per wavefront halve the LDS operand reads, which
-//                bound the kernel at one.  Few rows (W = 1, decode) are bound by streaming the
-//                cache: the key range is split until about four wavefronts per CU stream, each
-//                with a whole block (16 KB of K and of V at D = 128) in flight.
+//                Long prompts are bound by the matrix cores and the softmax's VALU work about
+//                equally, three wavefronts per SIMD overlapping them.  (Two query tiles per
+//                wavefront halve the LDS operand reads but leave two wavefronts per SIMD: 99
+//                against 91 us for 2048 tokens of 32 heads of 96.)  Few rows (W = 1, decode) are
+//                bound by streaming the cache: the key range is split until about four wavefronts
+//                per CU stream, each with a whole block (16 KB of K and of V at D = 128) in flight.
 //   gqa_combine  merges the split partials (max, sum, unnormalised O) into attn_output.
 #include <algorithm>
 #include <cmath>
@@ -88,6 +89,19 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const f16* p, uint32
 }
 __device__ __forceinline__ u32x4 buffer_load16(__amdgpu_buffer_rsrc_t r, uint32_t off, uint32_t soff) {
     return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, (int)soff, 0));
+}
+
+// v - h[I], exact to fp32: one mixed FMA instead of a conversion and a subtraction.
+template <int I>
+__device__ __forceinline__ float minus_half(float v, f16x2 h) {
+    float r;
+    if constexpr (I == 0)
+        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(as_u32(h)), "v"(v));
+    else
+        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]"
+            : "=v"(r)
+            : "v"(as_u32(h)), "v"(v));
+    return r;
 }
 
 // LDS row of key kk within a 64-key block: the 16 keys one score MFMA reads (see gqa_attend)
@@ -173,8 +187,8 @@ gqa_prep(const f16* __restrict__ qkv, const int32_t* __restrict__ seqlens,
         *reinterpret_cast<f16x8*>((is_v ? vn : kn) + (bk * g.S + s) * D + d0) = v;
 }
 
-// W wavefronts of QT 16-row query tiles each.
-template <int D, int W, int QT>
+// W wavefronts of 16 query rows each.
+template <int D, int W>
 __global__ void __launch_bounds__(64 * W) __attribute__((amdgpu_waves_per_eu(W == 1 ? 1 : 2)))
 gqa_attend(const f16* __restrict__ qr, const f16* __restrict__ past_k,
            const f16* __restrict__ past_v, const f16* __restrict__ kn,
@@ -221,8 +235,8 @@ gqa_attend(const f16* __restrict__ qr, const f16* __restrict__ past_k,
     const int b = (int)(bk / g.nkv);
 
     const int64_t past_len = past_len_of(seqlens, b, g);
-    const int64_t r0 = (int64_t)rb * 16 * QT * W;
-    const int64_t r_hi = std::min<int64_t>(r0 + 16 * QT * W, g.R);
+    const int64_t r0 = (int64_t)rb * 16 * W;
+    const int64_t r_hi = std::min<int64_t>(r0 + 16 * W, g.R);
     const int64_t key_end = past_len + (r_hi - 1) / g.G + 1;
     const int64_t k_begin = (int64_t)split * g.chunk;
     const int64_t k_stop = std::min<int64_t>(k_begin + g.chunk, key_end);
@@ -232,62 +246,45 @@ gqa_attend(const f16* __restrict__ qr, const f16* __restrict__ past_k,
     const int wave = tid >> 6;
     const int j = lane & 15;
     const int grp = lane >> 4;
-    const int64_t wr0 = r0 + 16 * QT * wave;             // the wavefront's first row
+    const int64_t wr0 = r0 + 16 * wave;                  // the wavefront's first row
     const bool wave_active = wr0 < g.R;
-    int64_t r[QT];
-    bool rvalid[QT];
-#pragma unroll
-    for (int u = 0; u < QT; ++u) {
-        r[u] = wr0 + 16 * u + j;
-        rvalid[u] = r[u] < g.R;
-    }
+    const int64_t r = wr0 + j;
+    const bool rvalid = r < g.R;
 
     if (k_begin >= k_stop) {                             // no keys in this split
+        if (!rvalid) return;
+        const int64_t prow = ((int64_t)split * (g.work / (g.splits * g.row_blocks)) + bk) * g.R + r;
 #pragma unroll
-        for (int u = 0; u < QT; ++u) {
-            if (!rvalid[u]) continue;
-            const int64_t prow = ((int64_t)split * (g.work / (g.splits * g.row_blocks)) + bk) * g.R + r[u];
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt)
-                *reinterpret_cast<f32x4*>(part_o + prow * D + 16 * dt + 4 * grp) = f32x4{0, 0, 0, 0};
-            if (grp == 0) {
-                part_ml[2 * prow] = kMasked;
-                part_ml[2 * prow + 1] = 0.f;
-            }
+        for (int dt = 0; dt < DT; ++dt)
+            *reinterpret_cast<f32x4*>(part_o + prow * D + 16 * dt + 4 * grp) = f32x4{0, 0, 0, 0};
+        if (grp == 0) {
+            part_ml[2 * prow] = kMasked;
+            part_ml[2 * prow + 1] = 0.f;
         }
         return;
     }
 
-    int64_t tp[QT], tp_lo[QT];                           // this lane's query, the tile's first
-    const int64_t tp_hi = past_len + (std::min<int64_t>(wr0 + 16 * QT - 1, g.R - 1)) / g.G;
+    const int64_t rc = rvalid ? r : g.R - 1;
+    const int64_t tp = past_len + rc / g.G;              // this lane's query, the wavefront's first
+    const int64_t tp_lo = past_len + std::min<int64_t>(wr0, g.R - 1) / g.G;   // and last
+    const int64_t tp_hi = past_len + (std::min<int64_t>(wr0 + 15, g.R - 1)) / g.G;
     // Q^T fragments (B operand of the score MFMA): query j, dims 32 ks + 8 grp .. + 7, as fp16
     // high and low parts (two MFMAs), so the scores carry the fp32 rotation of Q.
-    f16x8 qf[QT][2][KS];
+    f16x8 qf[2][KS];
 #pragma unroll
-    for (int u = 0; u < QT; ++u) {
-        const int64_t rc = rvalid[u] ? r[u] : g.R - 1;
-        tp[u] = past_len + rc / g.G;
-        tp_lo[u] = past_len + std::min<int64_t>(wr0 + 16 * u, g.R - 1) / g.G;
+    for (int hl = 0; hl < 2; ++hl) {
+        const f16* qrow = qr + hl * g.q_elems + (bk * g.R + rc) * D;
 #pragma unroll
-        for (int hl = 0; hl < 2; ++hl) {
-            const f16* qrow = qr + hl * g.q_elems + (bk * g.R + rc) * D;
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks)
-                qf[u][hl][ks] = rvalid[u] && (!TAIL || ks + 1 < KS || grp < 2)
-                                    ? *reinterpret_cast<const f16x8*>(qrow + 32 * ks + 8 * grp)
-                                    : f16x8{};
-        }
+        for (int ks = 0; ks < KS; ++ks)
+            qf[hl][ks] = rvalid && (!TAIL || ks + 1 < KS || grp < 2)
+                             ? *reinterpret_cast<const f16x8*>(qrow + 32 * ks + 8 * grp)
+                             : f16x8{};
     }
 
-    f32x4 oacc[QT][DT];
-    float m_run[QT], l_run[QT];
+    f32x4 oacc[DT];
+    float m_run = kMasked, l_run = 0.f;
 #pragma unroll
-    for (int u = 0; u < QT; ++u) {
-        m_run[u] = kMasked;
-        l_run[u] = 0.f;
-#pragma unroll
-        for (int dt = 0; dt < DT; ++dt) oacc[u][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
+    for (int dt = 0; dt < DT; ++dt) oacc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     const bool copy = g.copy_past && rb == 0;
     const f16* pk_base = past_k + bk * g.past_stride * D;
@@ -381,13 +378,12 @@ gqa_attend(const f16* __restrict__ qr, const f16* __restrict__ past_k,
         const int64_t kend = block_end(kb);
         // S^T tiles: c2 = 32-key half, a = 16-key MFMA tile.  Lane (j, grp) ends up with the
         // scores of query j and keys kb + 32 c2 + 8 grp + 4 a + i.
-        f32x4 sc[QT][2][2];
+        f32x4 sc[2][2];
 #pragma unroll
         for (int c2 = 0; c2 < 2; ++c2)
 #pragma unroll
             for (int a = 0; a < 2; ++a) {
-#pragma unroll
-                for (int u = 0; u < QT; ++u) sc[u][c2][a] = f32x4{0.f, 0.f, 0.f, 0.f};
+                sc[c2][a] = f32x4{0.f, 0.f, 0.f, 0.f};
                 const f16* krow = &Ks[(32 * c2 + 16 * a + j) * KP];
 #pragma unroll
                 for (int ks = 0; ks < KS; ++ks) {
@@ -404,66 +400,62 @@ gqa_attend(const f16* __restrict__ qr, const f16* __restrict__ past_k,
                     }
 #pragma unroll
                     for (int hl = 0; hl < 2; ++hl)
-#pragma unroll
-                        for (int u = 0; u < QT; ++u)
-                            sc[u][c2][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-                                kf, qf[u][hl][ks], sc[u][c2][a], 0, 0, 0);
+                        sc[c2][a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+                            kf, qf[hl][ks], sc[c2][a], 0, 0, 0);
                 }
             }
-        f16x8 pb[QT][2], pl[QT][2];                      // P = pb + pl to 2^-22
-#pragma unroll
-        for (int u = 0; u < QT; ++u) {
-            // uniform: the block crosses the diagonal, or is short
-            if (kb + kBN - 1 > tp_lo[u] || kend - kb < kBN) {
-                // first masked key of the lane, counted from its first key of the block
-                const int cut = (int)std::min<int64_t>(tp[u] + 1 - kb, kend - kb) - 8 * grp;
-#pragma unroll
-                for (int c2 = 0; c2 < 2; ++c2)
-#pragma unroll
-                    for (int a = 0; a < 2; ++a)
-#pragma unroll
-                        for (int i = 0; i < 4; ++i)
-                            if (32 * c2 + 4 * a + i >= cut) sc[u][c2][a][i] = -INFINITY;
-            }
-            float mloc = -INFINITY;
+        f16x8 pb[2], pl[2];                              // P = pb + pl to 2^-22
+        // uniform: the block crosses the diagonal, or is short
+        if (kb + kBN - 1 > tp_lo || kend - kb < kBN) {
+            // first masked key of the lane, counted from its first key of the block
+            const int cut = (int)std::min<int64_t>(tp + 1 - kb, kend - kb) - 8 * grp;
 #pragma unroll
             for (int c2 = 0; c2 < 2; ++c2)
 #pragma unroll
                 for (int a = 0; a < 2; ++a)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) mloc = fmaxf(mloc, sc[u][c2][a][i]);
-            mloc *= g.scale_log2;                        // positive: a masked score stays -inf
-            mloc = fmaxf(mloc, __shfl_xor(mloc, 16));
-            mloc = fmaxf(mloc, __shfl_xor(mloc, 32));
-            const float m_new = fmaxf(m_run[u], mloc);
-            // most blocks after the first few raise no row's maximum: nothing to rescale
-            if (__any(m_new != m_run[u])) {
-                const float alpha = __builtin_amdgcn_exp2f(m_run[u] - m_new);
-                m_run[u] = m_new;
-                l_run[u] *= alpha;
-#pragma unroll
-                for (int dt = 0; dt < DT; ++dt) oacc[u][dt] *= alpha;
-            }
-            float l = 0.f;
-#pragma unroll
-            for (int c2 = 0; c2 < 2; ++c2)
-#pragma unroll
-                for (int i = 0; i < 8; i += 2) {
-                    float p[2];
-#pragma unroll
-                    for (int e = 0; e < 2; ++e) {
-                        p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(
-                            sc[u][c2][i >> 2][(i & 3) + e], g.scale_log2, -m_new));
-                        l += p[e];
-                    }
-                    const f16x2 hi = {(f16)p[0], (f16)p[1]};
-                    pb[u][c2][i] = hi.x;
-                    pb[u][c2][i + 1] = hi.y;
-                    pl[u][c2][i] = (f16)__builtin_fmaf((float)hi.x, -1.f, p[0]);
-                    pl[u][c2][i + 1] = (f16)__builtin_fmaf((float)hi.y, -1.f, p[1]);
-                }
-            l_run[u] += l;
+                    for (int i = 0; i < 4; ++i)
+                        if (32 * c2 + 4 * a + i >= cut) sc[c2][a][i] = -INFINITY;
         }
+        float mloc = -INFINITY;
+#pragma unroll
+        for (int c2 = 0; c2 < 2; ++c2)
+#pragma unroll
+            for (int a = 0; a < 2; ++a)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) mloc = fmaxf(mloc, sc[c2][a][i]);
+        mloc *= g.scale_log2;                            // positive: a masked score stays -inf
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 16));
+        mloc = fmaxf(mloc, __shfl_xor(mloc, 32));
+        const float m_new = fmaxf(m_run, mloc);
+        // most blocks after the first few raise no row's maximum: nothing to rescale
+        if (__any(m_new != m_run)) {
+            const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+            m_run = m_new;
+            l_run *= alpha;
+#pragma unroll
+            for (int dt = 0; dt < DT; ++dt) oacc[dt] *= alpha;
+        }
+        float l = 0.f;
+#pragma unroll
+        for (int c2 = 0; c2 < 2; ++c2)
+#pragma unroll
+            for (int i = 0; i < 8; i += 2) {
+                float p[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e) {
+                    p[e] = __builtin_amdgcn_exp2f(__builtin_fmaf(
+                        sc[c2][i >> 2][(i & 3) + e], g.scale_log2, -m_new));
+                    l += p[e];
+                }
+                const f16x2 hi = {(f16)p[0], (f16)p[1]};
+                const f16x2 lo = {(f16)minus_half<0>(p[0], hi), (f16)minus_half<1>(p[1], hi)};
+                pb[c2][i] = hi.x;
+                pb[c2][i + 1] = hi.y;
+                pl[c2][i] = lo.x;
+                pl[c2][i + 1] = lo.y;
+            }
+        l_run += l;
         // O^T += V^T P^T over keys kb + 32 c2 + 8 grp .. + 7.
 #pragma unroll
         for (int c2 = 0; c2 < 2; ++c2)
@@ -471,12 +463,8 @@ gqa_attend(const f16* __restrict__ qr, const f16* __restrict__ past_k,
             for (int dt = 0; dt < DT; ++dt) {
                 const f16x8 vf =
                     *reinterpret_cast<const f16x8*>(&Vt[(16 * dt + j) * kVP + 32 * c2 + 8 * grp]);
-#pragma unroll
-                for (int u = 0; u < QT; ++u)
-                    oacc[u][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pb[u][c2], oacc[u][dt], 0, 0, 0);
-#pragma unroll
-                for (int u = 0; u < QT; ++u)
-                    oacc[u][dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl[u][c2], oacc[u][dt], 0, 0, 0);
+                oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pb[c2], oacc[dt], 0, 0, 0);
+                oacc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vf, pl[c2], oacc[dt], 0, 0, 0);
             }
     };
 
@@ -491,35 +479,32 @@ gqa_attend(const f16* __restrict__ qr, const f16* __restrict__ past_k,
         kb = next;
     }
 
+    float l = l_run;
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (!rvalid) return;
+    if (g.splits == 1) {
+        const int64_t s = r / g.G;
+        const int h = (int)(bk % g.nkv) * g.G + (int)(r % g.G);
+        f16* o = out + (((int64_t)b * g.S + s) * g.nq + h) * D + 4 * grp;
+        const float inv = 1.f / l;
 #pragma unroll
-    for (int u = 0; u < QT; ++u) {
-        float l = l_run[u];
-        l += __shfl_xor(l, 16);
-        l += __shfl_xor(l, 32);
-        if (!rvalid[u]) continue;
-        if (g.splits == 1) {
-            const int64_t s = r[u] / g.G;
-            const int h = (int)(bk % g.nkv) * g.G + (int)(r[u] % g.G);
-            f16* o = out + (((int64_t)b * g.S + s) * g.nq + h) * D + 4 * grp;
-            const float inv = 1.f / l;
-#pragma unroll
-            for (int dt = 0; dt < DT; ++dt) {
-                const f32x4 x = oacc[u][dt];
-                const h4 v = {(f16)(x[0] * inv), (f16)(x[1] * inv), (f16)(x[2] * inv),
-                              (f16)(x[3] * inv)};
-                *reinterpret_cast<h4*>(o + 16 * dt) = v;
-            }
-            continue;
+        for (int dt = 0; dt < DT; ++dt) {
+            const f32x4 x = oacc[dt];
+            const h4 v = {(f16)(x[0] * inv), (f16)(x[1] * inv), (f16)(x[2] * inv),
+                          (f16)(x[3] * inv)};
+            *reinterpret_cast<h4*>(o + 16 * dt) = v;
         }
-        const int64_t bks = g.work / ((int64_t)g.splits * g.row_blocks);
-        const int64_t prow = ((int64_t)split * bks + bk) * g.R + r[u];
+        return;
+    }
+    const int64_t bks = g.work / ((int64_t)g.splits * g.row_blocks);
+    const int64_t prow = ((int64_t)split * bks + bk) * g.R + r;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
-            *reinterpret_cast<f32x4*>(part_o + prow * D + 16 * dt + 4 * grp) = oacc[u][dt];
-        if (grp == 0) {
-            part_ml[2 * prow] = m_run[u];
-            part_ml[2 * prow + 1] = l;
-        }
+    for (int dt = 0; dt < DT; ++dt)
+        *reinterpret_cast<f32x4*>(part_o + prow * D + 16 * dt + 4 * grp) = oacc[dt];
+    if (grp == 0) {
+        part_ml[2 * prow] = m_run;
+        part_ml[2 * prow + 1] = l;
     }
 }
 
@@ -576,10 +561,7 @@ GqaPlan gqa_plan(const GqaArgs& a) {
     const int64_t R = a.seq * G;
     const int64_t bk = a.batch * a.nkv;
     p.waves = R > 16 ? 4 : 1;
-    // two query tiles per wavefront where 128-row blocks still give every CU a workgroup (and
-    // the registers hold both: head_dim up to 128)
-    p.qt = p.waves == 4 && a.d <= 128 && bk * ((R + 127) / 128) >= 256 ? 2 : 1;
-    const int64_t block = 16 * p.waves * p.qt;
+    const int64_t block = 16 * p.waves;
     p.row_blocks = (R + block - 1) / block;
     const int64_t base = bk * p.row_blocks;
     const int64_t t_max = a.past_stride + a.seq;        // bound on keys per query
@@ -589,7 +571,7 @@ GqaPlan gqa_plan(const GqaArgs& a) {
     // 512 of four wavefronts; at least one (four wavefronts: two) 64-key blocks each.
     const int64_t fill = p.waves == 1 ? 1024 : 512;
     const int64_t least = p.waves == 1 ? kBN : 2 * kBN;
-    if (p.qt == 1 && base < fill && t_max > least) {
+    if (base < fill && t_max > least) {
         const int64_t want = (fill + base - 1) / base;
         int64_t chunk = (t_max + want - 1) / want;
         chunk = std::max<int64_t>(least, (chunk + kBN - 1) / kBN * kBN);
@@ -612,11 +594,11 @@ size_t gqa_workspace_bytes(const GqaArgs& a) {
     return n;
 }
 
-template <int D, int W, int QT>
+template <int D, int W>
 static void attend_go(const GqaDims& g, const f16* qr, const void* pk, const void* pv,
                       const f16* kn, const f16* vn, const int32_t* seqlens, void* out, void* prk,
                       void* prv, float* po, float* pml, hipStream_t st) {
-    hipLaunchKernelGGL((gqa_attend<D, W, QT>), dim3((unsigned)g.work), dim3(64 * W), 0, st, qr,
+    hipLaunchKernelGGL((gqa_attend<D, W>), dim3((unsigned)g.work), dim3(64 * W), 0, st, qr,
                        static_cast<const f16*>(pk), static_cast<const f16*>(pv), kn, vn, seqlens,
                        static_cast<f16*>(out), static_cast<f16*>(prk), static_cast<f16*>(prv), po,
                        pml, g);
@@ -627,12 +609,8 @@ static void attend_w(const GqaPlan& p, const GqaDims& g, const f16* qr, const vo
                      const void* pv, const f16* kn, const f16* vn, const int32_t* seqlens,
                      void* out, void* prk, void* prv, float* po, float* pml, hipStream_t st) {
     if (p.waves == 1)
-        return attend_go<D, 1, 1>(g, qr, pk, pv, kn, vn, seqlens, out, prk, prv, po, pml, st);
-    if constexpr (D <= 128) {
-        if (p.qt == 2)
-            return attend_go<D, 4, 2>(g, qr, pk, pv, kn, vn, seqlens, out, prk, prv, po, pml, st);
-    }
-    attend_go<D, 4, 1>(g, qr, pk, pv, kn, vn, seqlens, out, prk, prv, po, pml, st);
+        return attend_go<D, 1>(g, qr, pk, pv, kn, vn, seqlens, out, prk, prv, po, pml, st);
+    attend_go<D, 4>(g, qr, pk, pv, kn, vn, seqlens, out, prk, prv, po, pml, st);
 }
 
 hipError_t launch_gqa(const GqaArgs& a, const void* qkv, const void* past_k, const void* past_v,

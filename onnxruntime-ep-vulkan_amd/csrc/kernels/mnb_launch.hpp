@@ -336,8 +336,7 @@ struct GqaArgs {
     bool copy_past;      // present is its own buffer: the past tokens are copied into it
 };
 struct GqaPlan {
-    int waves;           // wavefronts per workgroup
-    int qt;              // 16-row query tiles per wavefront
+    int waves;           // wavefronts per workgroup (16 query rows each)
     int splits;          // workgroups along the keys of one row block
     int64_t row_blocks;  // row blocks per (batch, KV head)
     int64_t chunk;       // keys per split (a multiple of 64)

@@ -106,11 +106,11 @@ def test_matches_oracle(cuda, B, S, past, Nq, Nkv, D):
 
 
 @pytest.mark.parametrize("B,S,past,Nq,Nkv,D", [
-    (4, 260, 40, 32, 32, 64),    # two query tiles per wavefront: 128-row blocks, the last of 4 rows
-    (3, 300, 0, 32, 32, 96),     # ... whole heads per XCD
-    (16, 65, 0, 64, 16, 128),    # ... 4 query heads per KV head
-    (5, 129, 3, 64, 32, 112),    # ... a 16-deep tail, workgroups not a multiple of 8
-    (2, 70, 5, 8, 8, 144),       # above 128 dims: one tile per wavefront
+    (4, 260, 40, 32, 32, 64),    # unsplit: 64-row blocks, the last of 4 rows; a past off a key block
+    (3, 300, 0, 32, 32, 96),     # whole heads per XCD, longest blocks first
+    (16, 65, 0, 64, 16, 128),    # 4 query heads per KV head
+    (5, 129, 3, 64, 32, 112),    # a half-empty last score step, workgroups not a multiple of 8
+    (2, 70, 5, 8, 8, 144),       # the same above 128 dims
     (1, 4, 4092, 4, 1, 128),     # 16 rows, 64 splits of one 64-key block
     (2, 2, 63, 8, 2, 96),        # splits that end on a block's edge
 ])
