@@ -58,6 +58,7 @@ HIP_SOURCES = [
     CSRC / "kernels" / "mnb_rows64_bs32.hip",
     CSRC / "kernels" / "mnb_rows64_bs64.hip",
     CSRC / "kernels" / "mnb_rows64_bs128.hip",
+    CSRC / "kernels" / "mnb_gemm_i8.hip",
     CSRC / "kernels" / "mnb_gemm.hip",
     CSRC / "kernels" / "mnb_group_gemv.hip",
     CSRC / "kernels" / "mnb_strip_gemv.hip",

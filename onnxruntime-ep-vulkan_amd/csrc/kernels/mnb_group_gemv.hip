@@ -740,6 +740,14 @@ hipError_t launch_acc4(const void* a, bool a_f16, const uint8_t* b, const void* 
         if (e != hipSuccess) return e;
         return launch_strip_gemv(sg, true, qa, sa, nullptr, nullptr, b, s, z, y, m, n, k, bs, st);
     }
+    GemmI8Geom ig;
+    if (a_f16 && !strip_gemv_forced_off() && reinterpret_cast<uintptr_t>(s) % 2 == 0 &&
+        gemm_i8_geometry(m, n, k, bits, bs, &ig)) {
+        hipError_t e = launch_quantize_a_int8(a, true, qa, sa, nullptr, true, m, k, bs, st, nullptr,
+                                              0, m);
+        if (e != hipSuccess) return e;
+        return launch_gemm_i8(ig, qa, sa, b, b_strips, s, z, y, m, n, k, bs, st);
+    }
     f32x4* part = g.ksplit > 1 ? reinterpret_cast<f32x4*>(ws + l.part) : nullptr;
     int* cnt = g.ksplit > 1 ? reinterpret_cast<int*>(ws + l.cnt) : nullptr;
     hipError_t e = launch_quantize_a_int8(a, a_f16, qa, sa, nullptr, true, m, k, bs, st, cnt,

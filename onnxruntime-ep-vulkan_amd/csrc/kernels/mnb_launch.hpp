@@ -116,6 +116,18 @@ hipError_t launch_gemm_direct_b8(int bs, const GemmConfig& c, const void* a, con
 hipError_t launch_splitk_sum(const float* part, void* y, int64_t mn, int ksplit,
                              hipStream_t stream);
 
+// accuracy_level 4 above 64 rows, fp16 scales and output, K % 64 == 0 (mnb_gemm_i8.hip):
+// qa are the quantiser's permuted codes [m][k], sa its scales block-major [k / bs][m]; b_strips:
+// the int8-order strip copy of B, read in place of b when not null.
+struct GemmI8Geom {
+    int bm, bn;          // workgroup tile, four wavefronts
+    int64_t tiles_m, tiles_n;
+};
+bool gemm_i8_geometry(int64_t m, int64_t n, int64_t k, int bits, int bs, GemmI8Geom* out);
+hipError_t launch_gemm_i8(const GemmI8Geom& c, const int8_t* qa, const float* sa,
+                          const uint8_t* b, const uint8_t* b_strips, const void* s,
+                          const uint8_t* z, void* y, int64_t m, int64_t n, int64_t k, int bs,
+                          hipStream_t stream);
 // 17 to 64 fp16 rows, int4, blocks of 32 to 128, K % 64 == 0 (mnb_rows64.hpp): s 16-column strips
 // and all the rows (mt 16-row tiles) per workgroup of eight wavefronts, K split over them.
 struct Rows64Geom {

@@ -185,6 +185,13 @@ static int plan_search(const mnb_problem* p, mnb_plan_info* out) {
             out->tile_m = 16;
             out->grid_x = ag.gx;
             out->grid_y = 1;
+        } else if (mnb::GemmI8Geom ig{}; f16 && forced_kernel() != MNB_KERNEL_GROUP_MFMA &&
+                   mnb::gemm_i8_geometry(p->m, p->n, p->k, p->bits, p->block_size, &ig)) {
+            out->waves_per_group = 4;
+            out->tile_n = ig.bn;
+            out->tile_m = ig.bm;
+            out->grid_x = ig.tiles_m * ig.tiles_n;
+            out->grid_y = 1;
         } else {
             const mnb::GroupGeom g =
                 mnb::group_geometry(p->m, p->n, p->k, 1, true, p->block_size, true);

@@ -140,6 +140,63 @@ def test_accuracy_level_4(cuda, M, N, K, bs, zp):
     assert orc.max_err_rms_normalised(y, ref) <= 6e-2
 
 
+# The int8 GEMM above 64 rows: 64- and 128-row tiles, rows and columns off a tile, a last half quad
+# (K % 128 == 64), odd quad counts, K / bs odd; both weight layouts.
+GEMM_I8 = [
+    (65, 8200, 576, 64, True, 64),
+    (100, 4100, 1088, 32, True, 64),
+    (257, 130, 320, 32, False, 64),
+    (300, 200, 1536, 128, True, 64),
+    (129, 4120, 1152, 32, False, 64),
+    (900, 8200, 192, 64, False, 128),
+    (1100, 7400, 320, 32, True, 128),
+    (961, 8184, 768, 64, True, 128),
+    (1024, 8200, 512, 128, False, 128),
+    (1030, 7300, 384, 128, True, 128),
+]
+
+
+@pytest.mark.parametrize("layout", ["ort", "strips"])
+@pytest.mark.parametrize("M,N,K,bs,zp,tile", GEMM_I8)
+def test_accuracy_level_4_gemm(cuda, M, N, K, bs, zp, tile, layout):
+    import ctypes as C
+    import mnb
+    import torch
+
+    p = mnb.problem(M, N, K, 4, bs, zp, mnb.DTYPE_F16, 4)
+    info = mnb.plan(p)
+    assert (info.kernel, info.tile_m, info.tile_n) == (mnb.KERNEL_ACC4_I8, tile, 128)
+    inp = orc.make_inputs(M, N, K, bits=4, block_size=bs, with_zp=zp, seed=M + N + K)
+    print(f"[gpu] acc4 gemm M={M} N={N} K={K} bs={bs} zp={zp} {layout}", flush=True)
+    A, B, S, Z = (_dev(inp[k], cuda) for k in ("A", "B", "scales", "zp"))
+    if layout == "ort":
+        y = mnb.matmul_nbits(A, B, S, Z, N, K, 4, bs, accuracy_level=4)
+    else:
+        lib, s, w = mnb.load(), C.c_void_p(), C.c_void_p()
+        mnb.check(lib.mnb_session_create(0, C.byref(s)))
+        z = inp["zp"]
+        mnb.check(lib.mnb_weights_upload(
+            s, C.byref(p), inp["B"].ctypes.data, inp["B"].nbytes, inp["scales"].ctypes.data,
+            inp["scales"].nbytes, z.ctypes.data if zp else None, z.nbytes if zp else 0, C.byref(w)))
+        rc = lib.mnb_weights_prepack(w, None)
+        y = torch.empty(M, N, dtype=torch.float16, device=cuda)
+        torch.cuda.synchronize()
+        if rc == mnb.MNB_OK:
+            mnb.check(lib.mnb_session_run(s, w, M, A.data_ptr(), 1, y.data_ptr(), 1))
+        mnb.check(lib.mnb_weights_release(w))
+        mnb.check(lib.mnb_session_destroy(s))
+        if rc == mnb.MNB_ERR_UNSUPPORTED:
+            pytest.skip("the node has no strip copy")
+        mnb.check(rc)
+    torch.cuda.synchronize()
+    # the level's definition: int8 codes and scales of A, then exact sums (the GPU's fp64 product)
+    qa, sa, _ = orc.quantize_a_int8(inp["A"], bs)
+    a = torch.from_numpy(qa.astype(np.float64) * np.repeat(sa.astype(np.float64), bs, axis=1)).to(cuda)
+    w64 = torch.from_numpy(orc.dequantize_f32(inp["B"], inp["scales"], inp["zp"], N, K, 4, bs)
+                           .astype(np.float64)).to(cuda)
+    _check(y.cpu().numpy(), (a @ w64.t()).cpu().numpy(), "acc4 gemm")
+
+
 def test_accuracy_level_4_split_k_reuses_workspace(cuda):
     # The row-tiled int8 GEMV (MNB_FORCE_KERNEL=group) hands partial tiles between workgroups
     # through the workspace and a counter per strip that the quantiser clears: three calls on one
