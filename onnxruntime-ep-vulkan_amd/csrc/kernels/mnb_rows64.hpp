@@ -10,7 +10,7 @@
 // wavefront w takes the w-th of eight contiguous runs of quads (128 k) of K, on its own from the
 // first load to the final sum: no barrier inside the loop, so the two wavefronts of a SIMD cover
 // each other's waits.  S makes the workgroups fit the 256 CUs in as few rounds as pay (see
-// rows64_strips).  The eight partial tiles are added in LDS in wavefront order.
+// rows64_geometry).  The eight partial tiles are added in LDS in wavefront order.
 //
 // Data movement.  A by LDS DMA into the wavefront's two stages of 64 k (8 rows x 128 bytes per
 // instruction: whole lines; 16-byte slot s of row r at s ^ (r & 7), so operand reads are free of
