@@ -1,5 +1,5 @@
 // Prefill MatMulNBits on gfx950: dequantise-into-LDS fp16 MFMA GEMM (fp16 A; 4- or 8-bit
-// weights; blocks of 16, 32, 64 or 128).
+// weights in blocks of 16; larger blocks go to mnb_gemm_direct.hpp), and the tile choice of both.
 //
 // Work split.  One workgroup of 8 wavefronts owns a 256 x 128 tile of Y; the wavefronts form a
 // 4 (M) x 2 (N) grid and each owns a 64 x 64 sub-tile of four 32 x 32 MFMA tiles.  K is walked in
@@ -30,8 +30,7 @@
 // kernel's per-block fp32 partial (rust/shaders/glsl/templates/q_gemv.comp:571-579) -- and added
 // to the tile's accumulator scaled by the block's scale.  The scaled add of one sub-block is
 // spread between the MFMAs of the next, so that it runs on the VALU while the matrix core works.
-// Blocks of 16 are one MFMA each; blocks of 64 or 128 scale the partial of each 64-k step on
-// its own (the same scale twice for a 128 block).
+// Blocks of 16 are one MFMA each.
 #include <algorithm>
 #include <type_traits>
 

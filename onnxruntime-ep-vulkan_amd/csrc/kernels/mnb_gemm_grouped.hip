@@ -1,8 +1,8 @@
 // The prefill GEMM of mnb_gemm_direct.hpp over the experts of a mixture of experts: every expert's
 // rows times its own int4 weights in one launch.
 //
-// Tiles of 128 rows x 192 columns (128 for blocks of 64 and 128), as many row tiles as the experts' row counts need; a tile with
-// at most 64 or 32 rows multiplies only those quarters, so an expert's last tile costs what its
+// Tiles of 128 rows x 192 columns (128 for blocks of 64 and 128), as many row tiles as the experts'
+// row counts need; a tile with at most 64 or 32 rows multiplies only those quarters, so an expert's last tile costs what its
 // rows cost (1024 tokens over 32 experts, 4 each: 128 rows per expert on average, half of the
 // experts with a few rows in a second tile).
 #include "mnb_gemm_direct.hpp"
